@@ -11,6 +11,7 @@
 #include "kernels.h"
 #include "staging.h"
 #include "vti.h"
+#include "walk.h"
 
 namespace nmk {
 
@@ -40,10 +41,10 @@ struct DevBuf {
             else (void)hipFree(ptr);
         }
         ptr = nullptr;
+        count = 0;
     }
     void alloc(size_t n) {
         release();
-        count = 0;
         if (!n) return;
         if (source) ptr = static_cast<P *>(source->allocate(n * sizeof(P)));
         else HIPCHK(hipMalloc((void **)&ptr, n * sizeof(P)));
@@ -141,6 +142,24 @@ int pow2_at_least(int v) {
     return p;
 }
 
+// Launch shape of the walking solvers for lines of M points, Mt of them per
+// component and propagation: chunks of at most 8 points (16 spill), as many as
+// bring the threads of a launch to 128 K, up to 64; as many lines per block as
+// fit 512 threads of both components, up to 8.  W = 0: no shape (lines over
+// 1024 or under 16 points).
+WalkShape walk_shape(int M, int Mt, int nprops) {
+    WalkShape sh{};
+    if (M > 1024) return sh;
+    const int64_t lines = (int64_t)Mt * 2 * nprops;
+    int par = 1;
+    while (par < 64 && (int64_t)par * lines < 131072) par *= 2;
+    sh.lp = make_line_plan(M, std::max(16, std::max(pow2_at_least((M + 7) / 8), par)));
+    for (sh.W = 8; sh.W > 1; sh.W /= 2)
+        if (2 * sh.W * sh.lp.P <= 512 && sh.W * sh.lp.P % 64 == 0) return sh;
+    sh.W = 0;
+    return sh;
+}
+
 template <class T>
 class RunnerT final : public Runner {
 public:
@@ -154,7 +173,7 @@ public:
         }
         sz_ = sizes_of(p, o);
         bind_source(o.allocator, bulk_, bt_, lc_, weights_, q_, iso_t_, iso_n_, partials_, mask_, twx_, twy_, E_, sp_, pp_, cf_,
-                    xt_, fb_[0], fb_[1], fb_[2], fb_[3], flag_);
+                    xt_, fb_[0], fb_[1], fb_[2], fb_[3], flag_, mat_, phase_);
         g_.Nx = p.Nx;
         g_.Ny = p.Ny;
         g_.Nz = p.Nz;
@@ -190,8 +209,7 @@ public:
         sp_.alloc(sz_.nslots_max);
         pp_.alloc(sz_.nprops_max);
         partials_.alloc((size_t)kNrefBlocks * sz_.nslots_max);
-        cf_.alloc((size_t)sz_.ring * sz_.nslots_max * cf_slot_size(g_.Mx, g_.My));
-        set_tuning(o.tuning.x_chunks > 0 ? o.tuning : default_tuning(o.precision, g_.Mx, g_.My, sz_.nprops_max));
+        set_tuning(o.tuning);
         for (auto &b : fb_) b.alloc((size_t)sz_.nprops_max * 2 * sz_.NP);
         if (!dev_in) E_.alloc((size_t)sz_.nwl * sz_.nq * 4 * sz_.Nfull);
         if (p.bulk) {
@@ -274,7 +292,7 @@ public:
         size_t b = lc_.footprint() + weights_.footprint() + q_.footprint() + iso_t_.footprint() + iso_n_.footprint() +
                    partials_.footprint() + mask_.footprint() + twx_.footprint() + twy_.footprint() +
                    E_.footprint() + sp_.footprint() + pp_.footprint() + cf_.footprint() + xt_.footprint() +
-                   bulk_.footprint() + bt_.footprint() + flag_.footprint();
+                   bulk_.footprint() + bt_.footprint() + flag_.footprint() + mat_.footprint() + phase_.footprint();
         for (auto &f : fb_) b += f.footprint();
         return (int64_t)b;
     }
@@ -373,7 +391,11 @@ private:
     std::vector<c64> htwx_, htwy_;
     DevBuf<SlotParams> sp_;
     DevBuf<PropParams> pp_;
-    DevBuf<C2<T>> cf_, xt_;
+    DevBuf<C2<T>> cf_, xt_;        // stored stencils and x-line rows
+    DevBuf<c64> mat_;              // slab material, both axis orders (walking solvers)
+    DevBuf<C2<T>> phase_;          // phase operators beside it
+    bool walk_ = false;            // the walking solvers march
+    WalkShape wx_{}, wy_{};
     DevBuf<C2<T>> fb_[4];
     DevBuf<c64> bulk_;   // bulk output planes (p.bulk)
     // inputs and output as the kernels see them: the runner's own buffers, or
@@ -460,6 +482,11 @@ private:
             sp.ea = sp.ne * sp.ne - sp.eperp;
             sp.ehost = sp.nhost * sp.nhost;
             sp.alpha_im = p.ne_imag[w] / (p.ne[w] - p.no[w]);  // NaN/inf when ne == no, as the reference
+            sp.rx2 = 0.125 * sp.dZ / (sp.dX * sp.dX);
+            sp.ry2 = 0.125 * sp.dZ / (sp.dY * sp.dY);
+            sp.rxy = 0.03125 * sp.dZ / (sp.dX * sp.dY);
+            sp.gx = 0.0625 * sp.dZ / sp.dX;
+            sp.gy = 0.0625 * sp.dZ / sp.dY;
             sp.nin = p.nin[w];
             sp.nout_fresnel = p.nout_fresnel[w];
             sp.nout_filter = p.nout[w];
@@ -526,10 +553,10 @@ private:
             C2<T> *F = fb_[0].ptr;
             if (p.beam == BeamKind::None) {
                 const c64 *Ein = E_p_ + (size_t)w0 * sz_.nq * 4 * sz_.Nfull;
-                launch_pack_fields<T>(Ein, g_, pp_.ptr, nprops, sz_.nq, F, st_);
+                launch_pack_fields<T>(Ein, g_, pp_.ptr, nprops, sz_.nq, F, walk_, st_);
             } else {
                 launch_init_fields<T>(lc_p_, mask_p_, g_, sp_.ptr, pp_.ptr, nprops,
-                                      p.beam == BeamKind::Gaussian ? 1 : 0, p.waist, p.dx, p.dy, F, st_);
+                                      p.beam == BeamKind::Gaussian ? 1 : 0, p.waist, p.dx, p.dy, F, walk_, st_);
             }
         });
     }
@@ -580,12 +607,16 @@ private:
     // stream (an autotuner option) slab k+2's are computed while slab k
     // marches, and the boundary joins the two streams (about 10 us per join).
     C2<T> *march_launches(int nslots, int nprops) {
-        const int nsl = p_.Nz - 1, nw = p_.n_woodbury, R = sz_.ring, CB = sz_.coef_batch;
+        const int nsl = p_.Nz - 1, R = sz_.ring, CB = sz_.coef_batch;
         const size_t cfsz = (size_t)sz_.nslots_max * cf_slot_size(g_.Mx, g_.My);
         const size_t xtsz = xt_.count / R;
-        auto CF = [&](int k) { return cf_.ptr + (size_t)(k % R) * cfsz; };
-        auto XT = [&](int k) { return xt_.ptr ? xt_.ptr + (size_t)(k % R) * xtsz : nullptr; };
-        const bool overlap = st2_ != nullptr && !tune_.coef_serial;
+        // what the boundary reads of slab k: its coefficient tiles, or its phase planes
+        auto CF = [&](int k) {
+            return walk_ ? phase_.ptr + (size_t)(k % R) * (size_t)sz_.nslots_max * 3 * sz_.NP
+                         : cf_.ptr + (size_t)(k % R) * cfsz;
+        };
+        const bool overlap = st2_ != nullptr && !walk_ && !tune_.coef_serial;
+        const WalkRing<T> ring = walk_ring();
         hipStream_t cs = overlap ? st2_ : st_;
         size_t evn = 0;
         auto record = [&](hipStream_t s) {
@@ -598,6 +629,10 @@ private:
         // coefficients of slabs k0 .. k0+n-1 in one launch on stream s
         auto coefs = [&](int k0, int n, hipStream_t s) {
             timed(KF_COEFS, [&] {
+                if (walk_) {
+                    launch_slab_material<T>(lc_p_, mask_p_, w_p_, g_, sp_.ptr, nslots, k0, n, ring, R, s);
+                    return;
+                }
                 launch_slab_coefs<T>(lc_p_, mask_p_, w_p_, g_, sp_.ptr, nslots, k0, n, cf_.ptr, (int64_t)cfsz,
                                      xt_.ptr, (int64_t)xtsz, R, lpx_, s);
             });
@@ -626,6 +661,49 @@ private:
         }
 
         C2<T> *cur = fb_[1].ptr, *other = fb_[0].ptr, *A = fb_[2].ptr, *B = fb_[3].ptr;
+        if (ready[0]) HIPCHK(hipStreamWaitEvent(st_, ready[0], 0));
+        // bulk plane 0: the entrance fields after the input interface
+        if (bulk_.ptr) {
+            const int beam = p_.beam == BeamKind::None ? 2 : p_.beam == BeamKind::Gaussian ? 1 : 0;
+            launch_bulk_entrance(lc_p_, mask_p_, g_, sp_.ptr, pp_.ptr, nprops, beam, p_.waist, p_.dx, p_.dy,
+                                 E_p_, sz_.nq, bulk_.ptr, st_);
+        }
+        timed(KF_BOUNDARY, [&] { launch_boundary<T>(other, cur, nullptr, CF(0), g_, pp_.ptr, nprops, 1, unshifted_[1], walk_, st_); });
+        for (int k = 0; k < nsl; k++) {
+            if (walk_) walk_slab(k, nslots, nprops, cur, other, A, B, ring);
+            else planes_slab(k, nprops, cur, other, A, B, CF(k));
+            // bulk plane k+1: the step's closing P_k, Sh applied to a copy
+            if (bulk_.ptr) {
+                launch_boundary<T>(cur, bt_.ptr, CF(k), nullptr, g_, pp_.ptr, nprops, 1, unshifted_[1], walk_, st_);
+                launch_bulk_plane<T>(bt_.ptr, g_, sp_.ptr, pp_.ptr, nprops, k + 1, sz_.nq, bulk_.ptr, walk_, st_);
+            }
+            // P_k, Sh | Sh, P_{k+1}
+            if (k + 1 < nsl) {
+                // coefficients on the march stream: the batch that starts at slab k+1 is
+                // computed here, just before the boundary and the slabs that read it (so
+                // it is still in the Infinity Cache), into the buffers of the batch before
+                // the current one, whose last reader has run
+                if (!overlap && (k + 1) % CB == 0) coefs(k + 1, std::min(CB, nsl - k - 1), st_);
+                if (ready[k + 1]) HIPCHK(hipStreamWaitEvent(st_, ready[k + 1], 0));
+                timed(KF_BOUNDARY, [&] { launch_boundary<T>(cur, other, CF(k), CF(k + 1), g_, pp_.ptr, nprops, 2, unshifted_[2], walk_, st_); });
+            } else {
+                timed(KF_BOUNDARY, [&] { launch_boundary<T>(cur, other, CF(k), nullptr, g_, pp_.ptr, nprops, 1, unshifted_[1], walk_, st_); });
+            }
+            std::swap(cur, other);
+            if (overlap && k + 2 < nsl) {
+                // CF(k) and XT(k) are free once the boundary above has run
+                HIPCHK(hipStreamWaitEvent(cs, record(st_), 0));
+                ready[k + 2] = coef(k + 2);
+            }
+        }
+        if (overlap) HIPCHK(hipStreamWaitEvent(st_, record(cs), 0));
+        return cur;
+    }
+
+    // both half-steps of slab k on its stored stencils cf: cur -> cur (y slow)
+    void planes_slab(int k, int nprops, C2<T> *cur, C2<T> *other, C2<T> *A, C2<T> *B, const C2<T> *cf) {
+        const int nw = p_.n_woodbury;
+        const C2<T> *xt = xt_.ptr ? xt_.ptr + (size_t)(k % sz_.ring) * (xt_.count / sz_.ring) : nullptr;
         // XCD work order (measured): a lone polarisation pair shares L2 best
         // across the two components; batches whose field planes total up to
         // about 32 MiB do best with the pairs innermost (the wavevectors of a
@@ -640,73 +718,87 @@ private:
                          : plane_bytes <= (size_t(32) << 20) ? 6
                          : sizeof(T) == 8 ? 10 : 0;
         const int ord = ord0 | (sz_.nq << 4);  // group size of order bit 3: the pairs of one slot
-        if (ready[0]) HIPCHK(hipStreamWaitEvent(st_, ready[0], 0));
-        // bulk plane 0: the entrance fields after the input interface
-        if (bulk_.ptr) {
-            const int beam = p_.beam == BeamKind::None ? 2 : p_.beam == BeamKind::Gaussian ? 1 : 0;
-            launch_bulk_entrance(lc_p_, mask_p_, g_, sp_.ptr, pp_.ptr, nprops, beam, p_.waist, p_.dx, p_.dy,
-                                 E_p_, sz_.nq, bulk_.ptr, st_);
-        }
-        timed(KF_BOUNDARY, [&] { launch_boundary<T>(other, cur, nullptr, CF(0), g_, pp_.ptr, nprops, 1, unshifted_[1], st_); });
-        for (int k = 0; k < nsl; k++) {
-            // x half-steps: other = (I - mu A_x)^-1 (I + mu A_y) cur by its Neumann series
-            // y0 + y1 + ... + y_nw: y0 goes to A, the first Neumann launch adds it to y1
-            // into other, the last one writes only the sum (in place)
-            if (g_.px) {
+        // x half-steps: other = (I - mu A_x)^-1 (I + mu A_y) cur by its Neumann series
+        // y0 + y1 + ... + y_nw: y0 goes to A, the first Neumann launch adds it to y1
+        // into other, the last one writes only the sum (in place)
+        if (g_.px) {
+            timed(KF_SOLVE_X, [&] {
+                launch_xsolve<T>(0, cur, nw > 0 ? A : other, nullptr, nullptr, cf, xt, g_, pp_.ptr, nprops, lpx_, tune_.x_rows, ord, tune_.lean, tune_.x_both & 1, st_);
+            });
+            C2<T> *a = A, *b = B;
+            for (int it = 0; it < nw; it++) {
                 timed(KF_SOLVE_X, [&] {
-                    launch_xsolve<T>(0, cur, nw > 0 ? A : other, nullptr, nullptr, CF(k), XT(k), g_, pp_.ptr, nprops, lpx_, tune_.x_rows, ord, tune_.lean, tune_.x_both & 1, st_);
+                    launch_xsolve<T>(1, a, it + 1 < nw ? b : nullptr, it == 0 ? a : other, other, cf, xt, g_, pp_.ptr, nprops, lpx_, tune_.x_rows, ord, tune_.lean, (tune_.x_both >> 1) & 1, st_);
                 });
-                C2<T> *a = A, *b = B;
-                for (int it = 0; it < nw; it++) {
-                    timed(KF_SOLVE_X, [&] {
-                        launch_xsolve<T>(1, a, it + 1 < nw ? b : nullptr, it == 0 ? a : other, other, CF(k), XT(k), g_, pp_.ptr, nprops, lpx_, tune_.x_rows, ord, tune_.lean, (tune_.x_both >> 1) & 1, st_);
-                    });
-                    std::swap(a, b);
-                }
-            } else {
-                timed(KF_EXPLICIT, [&] { launch_explicit<T>(1, cur, other, CF(k), g_, pp_.ptr, nprops, st_); });
+                std::swap(a, b);
             }
-            // y half-steps: cur = (I - mu A_y)^-1 (I + mu A_x) other by its Neumann series
-            if (g_.py) {
+        } else {
+            timed(KF_EXPLICIT, [&] { launch_explicit<T>(1, cur, other, cf, g_, pp_.ptr, nprops, st_); });
+        }
+        // y half-steps: cur = (I - mu A_y)^-1 (I + mu A_x) other by its Neumann series
+        if (g_.py) {
+            timed(KF_SOLVE_Y, [&] {
+                launch_ysolve<T>(0, other, nw > 0 ? A : cur, nullptr, nullptr, cf, g_, pp_.ptr, nprops, lpy_, tune_.y_cols, ord, tune_.lean, tune_.y_pair, st_);
+            });
+            C2<T> *a = A, *b = B;
+            for (int it = 0; it < nw; it++) {
                 timed(KF_SOLVE_Y, [&] {
-                    launch_ysolve<T>(0, other, nw > 0 ? A : cur, nullptr, nullptr, CF(k), g_, pp_.ptr, nprops, lpy_, tune_.y_cols, ord, tune_.lean, tune_.y_pair, st_);
+                    launch_ysolve<T>(1, a, it + 1 < nw ? b : nullptr, it == 0 ? a : cur, cur, cf, g_, pp_.ptr, nprops, lpy_, tune_.y_cols, ord, tune_.lean, tune_.y_pair, st_);
                 });
-                C2<T> *a = A, *b = B;
+                std::swap(a, b);
+            }
+        } else {
+            timed(KF_EXPLICIT, [&] { launch_explicit<T>(0, other, cur, cf, g_, pp_.ptr, nprops, st_); });
+        }
+    }
+
+    // material values of one ring buffer
+    size_t mat_slab() const { return (size_t)sz_.nslots_max * 2 * walk_points(g_.Mx, g_.My) * 5; }
+
+    WalkRing<T> walk_ring() const {
+        WalkRing<T> r{};
+        if (!walk_) return r;
+        r.mat = mat_.ptr;
+        r.mat_stride = mat_slab();
+        r.phase = phase_.ptr;
+        r.phase_stride = (size_t)sz_.nslots_max * 3 * sz_.NP;
+        return r;
+    }
+
+    // both half-steps of slab k with the walking solvers: cur (x slow) -> cur (x slow).  Lines along x read and
+    // write x slow, lines along y y slow; the launch that completes a half-step writes the other order, into a
+    // buffer that no block of it reads.
+    void walk_slab(int k, int nslots, int nprops, C2<T> *cur, C2<T> *other, C2<T> *A, C2<T> *B,
+                   const WalkRing<T> &ring) {
+        if constexpr (sizeof(T) == 8) {
+            const int nw = p_.n_woodbury;
+            const size_t b = (size_t)(k % sz_.ring);
+            WalkMaterial wm;
+            wm.nat = ring.mat + b * ring.mat_stride;
+            wm.tr = wm.nat + (size_t)nslots * walk_points(g_.Mx, g_.My) * 5;
+            C2<T> *in = cur;
+            for (int axis = 0; axis < 2; axis++) {
+                const WalkShape &sh = axis == 0 ? wx_ : wy_;
+                const int fam = axis == 0 ? KF_SOLVE_X : KF_SOLVE_Y;
+                // y0 + y1 + ... + y_nw: y0 goes to A, the first Neumann launch adds it to y1, the last one writes only
+                // the sum
+                C2<T> *done = nw > 0 ? cur : axis == 0 ? other : cur;
+                timed(fam, [&] {
+                    launch_walk(axis, 0, in, nw > 0 ? A : nullptr, nullptr, nw > 0 ? nullptr : done, nw == 0, wm, g_,
+                                sp_.ptr, pp_.ptr, nprops, 2 * sz_.nq, sh, st_);
+                });
+                C2<T> *a = A, *bb = B;
                 for (int it = 0; it < nw; it++) {
-                    timed(KF_SOLVE_Y, [&] {
-                        launch_ysolve<T>(1, a, it + 1 < nw ? b : nullptr, it == 0 ? a : cur, cur, CF(k), g_, pp_.ptr, nprops, lpy_, tune_.y_cols, ord, tune_.lean, tune_.y_pair, st_);
+                    const bool last = it + 1 == nw;
+                    timed(fam, [&] {
+                        launch_walk(axis, 1, a, last ? nullptr : bb, it == 0 ? a : other, last ? done : other, last, wm,
+                                    g_, sp_.ptr, pp_.ptr, nprops, 2 * sz_.nq, sh, st_);
                     });
-                    std::swap(a, b);
+                    std::swap(a, bb);
                 }
-            } else {
-                timed(KF_EXPLICIT, [&] { launch_explicit<T>(0, other, cur, CF(k), g_, pp_.ptr, nprops, st_); });
-            }
-            // bulk plane k+1: the step's closing P_k, Sh applied to a copy
-            if (bulk_.ptr) {
-                launch_boundary<T>(cur, bt_.ptr, CF(k), nullptr, g_, pp_.ptr, nprops, 1, unshifted_[1], st_);
-                launch_bulk_plane<T>(bt_.ptr, g_, sp_.ptr, pp_.ptr, nprops, k + 1, sz_.nq, bulk_.ptr, st_);
-            }
-            // P_k, Sh | Sh, P_{k+1}
-            if (k + 1 < nsl) {
-                // coefficients on the march stream: the batch that starts at slab k+1 is
-                // computed here, just before the boundary and the slabs that read it (so
-                // it is still in the Infinity Cache), into the buffers of the batch before
-                // the current one, whose last reader has run
-                if (!overlap && (k + 1) % CB == 0) coefs(k + 1, std::min(CB, nsl - k - 1), st_);
-                if (ready[k + 1]) HIPCHK(hipStreamWaitEvent(st_, ready[k + 1], 0));
-                timed(KF_BOUNDARY, [&] { launch_boundary<T>(cur, other, CF(k), CF(k + 1), g_, pp_.ptr, nprops, 2, unshifted_[2], st_); });
-            } else {
-                timed(KF_BOUNDARY, [&] { launch_boundary<T>(cur, other, CF(k), nullptr, g_, pp_.ptr, nprops, 1, unshifted_[1], st_); });
-            }
-            std::swap(cur, other);
-            if (overlap && k + 2 < nsl) {
-                // CF(k) and XT(k) are free once the boundary above has run
-                HIPCHK(hipStreamWaitEvent(cs, record(st_), 0));
-                ready[k + 2] = coef(k + 2);
+                in = done;
             }
         }
-        if (overlap) HIPCHK(hipStreamWaitEvent(st_, record(cs), 0));
-        return cur;
     }
 
     void drop_graphs() {
@@ -717,12 +809,37 @@ private:
         graphs_.clear();
     }
 
-    // validates t, then switches to it (the runner keeps its state when t is
-    // refused).  The captured graphs hold the buffer pointers of the old
-    // shapes, so they are destroyed before any buffer changes; a larger x-line
-    // row buffer is allocated beside the old one and swapped in only once the
-    // allocation has succeeded.
-    void set_tuning(const Tuning &t) {
+    // Validates the shapes asked for, then switches to them (the runner keeps
+    // its state when they are refused).  The captured graphs hold the buffer
+    // pointers of the old shapes, so they are destroyed before any buffer
+    // changes.
+    //
+    // FP64 marches at the built-in shapes take the walking solvers wherever
+    // they have a shape (both axes periodic, march lines of 16 to 1024
+    // points): 25.1 -> 17.2 ms for 512^2 x 100 at one propagation pair, 267.5
+    // -> 171.5 ms for 1024^2 x 200, 22.6 -> 21.1 ms for a 128^2 x 40 call at
+    // 7 pairs, even at 64^2 (1.25 ms).  Explicit shapes are shapes of the
+    // solvers on stored stencils; FP32 stays there too, where the stencils are
+    // half the bytes and the walk's FP64 arithmetic is not.
+    void set_tuning(const Tuning &asked) {
+        const bool builtin = asked.x_chunks <= 0;
+        WalkShape wx{}, wy{};
+        if (sizeof(T) == 8 && builtin && g_.px && g_.py) {
+            wx = walk_shape(g_.Mx, g_.My, sz_.nprops_max);
+            wy = walk_shape(g_.My, g_.Mx, sz_.nprops_max);
+        }
+        if (wx.W > 0 && wy.W > 0) {
+            drop_graphs();
+            cf_.release();
+            xt_.release();
+            alloc_walk();
+            walk_ = true;
+            wx_ = wx;
+            wy_ = wy;
+            tune_ = asked;
+            return;
+        }
+        const Tuning t = builtin ? default_tuning(o_.precision, g_.Mx, g_.My, sz_.nprops_max) : asked;
         const LinePlan lx = g_.px ? make_line_plan(g_.Mx, t.x_chunks) : lpx_;
         const LinePlan ly = g_.py ? make_line_plan(g_.My, t.y_chunks) : lpy_;
         if (g_.px && ((t.x_both ? 4 : 2) * lx.P * t.x_rows > 512 ||
@@ -732,31 +849,51 @@ private:
                       ysolve_lds_bytes<T>(ly, t.y_cols, t.y_pair) > max_block_lds()))
             throw std::runtime_error("y line solver tuning exceeds the block limits");
         drop_graphs();
-        if (g_.px) {
-            const size_t need = (size_t)sz_.ring * sz_.nslots_max * 2 * 3 * g_.My * lx.lmax * lx.P;
-            if (need > xt_.count) {
-                DevBuf<C2<T>> grown;
-                grown.source = xt_.source;
-                grown.alloc(need);  // throws with xt_ untouched
-                xt_.swap(grown);    // the old rows are released with `grown`
+        mat_.release();
+        phase_.release();
+        try {
+            if (!cf_.ptr) cf_.alloc((size_t)sz_.ring * sz_.nslots_max * cf_slot_size(g_.Mx, g_.My));
+            if (g_.px) {
+                // a larger x-line row buffer is allocated beside the old one
+                const size_t need = (size_t)sz_.ring * sz_.nslots_max * 2 * 3 * g_.My * lx.lmax * lx.P;
+                if (need > xt_.count) {
+                    DevBuf<C2<T>> grown;
+                    grown.source = xt_.source;
+                    grown.alloc(need);
+                    xt_.swap(grown);  // the old rows are released with `grown`
+                }
             }
+        } catch (...) {
+            if (walk_) {
+                cf_.release();
+                xt_.release();
+                alloc_walk();
+            }
+            throw;
         }
+        walk_ = false;
         tune_ = t;
         lpx_ = lx;
         lpy_ = ly;
     }
 
+    void alloc_walk() {
+        if (mat_.ptr) return;
+        mat_.alloc((size_t)sz_.ring * mat_slab());
+        phase_.alloc((size_t)sz_.ring * sz_.nslots_max * 3 * sz_.NP);
+    }
+
     void retune(const Tuning &t) override {
         HIPCHK(hipStreamSynchronize(st_));
         if (st2_) HIPCHK(hipStreamSynchronize(st2_));
-        set_tuning(t.x_chunks > 0 ? t : default_tuning(o_.precision, g_.Mx, g_.My, sz_.nprops_max));
+        set_tuning(t);
     }
 
     void output_batch(int w0, int nslots, int nprops, const C2<T> *state) {
         c64 *Eb = E_p_ + (size_t)w0 * sz_.nq * 4 * sz_.Nfull;
         timed(KF_OUTPUT, [&] {
             if (p_.Nz > 1) {
-                launch_output<T>(state, lc_p_, mask_p_, g_, sp_.ptr, pp_.ptr, nprops, sz_.nq, Eb, st_);
+                launch_output<T>(state, lc_p_, mask_p_, g_, sp_.ptr, pp_.ptr, nprops, sz_.nq, Eb, walk_, st_);
             } else {
                 const int beam = p_.beam == BeamKind::None ? 2 : p_.beam == BeamKind::Gaussian ? 1 : 0;
                 launch_output_entrance(lc_p_, mask_p_, g_, sp_.ptr, pp_.ptr, nprops, beam, p_.waist, p_.dx, p_.dy, Eb,
@@ -831,7 +968,9 @@ Tuning default_tuning(int precision, int Mx, int My, int nprops) {
 }
 
 int64_t estimate_footprint(const Problem &p, const Options &o) {
-    // mirrors the allocations of RunnerT, buffer by buffer
+    // mirrors the allocations of RunnerT, buffer by buffer; the line solvers'
+    // at the stored stencils' size, of which the walking solvers' material and
+    // phase operators are less than half
     check_mesh_limits(p, o);
     const Sizes s = sizes_of(p, o);
     const int64_t fsz = o.precision == 32 ? 8 : 16;

@@ -33,20 +33,45 @@ void launch_slab_coefs(const double *lc, const uint8_t *mask, const double *weig
                        const SlotParams *sp, int nslots, int iz0, int nz, C2<T> *cf, int64_t cfstride, C2<T> *xt,
                        int64_t xtstride, int ring, const LinePlan &lpx, hipStream_t st);
 
+// Ring of slab buffers of the solvers that generate the stencils from the
+// material (walk.h).  Per buffer: the nine slab averages of each point as five
+// 16-byte values, members named along (l) and across (t) the lines,
+//   (kll, klt) (ktt, ill) (ilt, itt) (1/eps_zz, vt) (vl, 0)
+// once as [y][x] for lines along y and once as [x][y] for lines along x, with
+// the mesh's duplicate column and row as point Mx and row My (the material of
+// column / row 0, 1/eps_zz of the duplicate: all that the march reads there);
+// and the phase operators, three planes per slot as [x][y]
+__host__ __device__ __forceinline__ size_t walk_points(int Mx, int My) { return (size_t)(Mx + 1) * (My + 1); }
+template <class T>
+struct WalkRing {
+    c64 *mat;
+    C2<T> *phase;
+    size_t mat_stride, phase_stride;
+};
+// slab material of slabs iz0 .. iz0+nz-1 into buffers iz % ring, one launch
+template <class T>
+void launch_slab_material(const double *lc, const uint8_t *mask, const double *weights, const Geo &g,
+                          const SlotParams *sp, int nslots, int iz0, int nz, const WalkRing<T> &wr, int ring,
+                          hipStream_t st);
+
+// x_slow (this and the launchers below): the march state is kept with x slow
+// ([x][y]) instead of y slow
+
 // input beam + input Fresnel (beam != None) or packing of caller fields
 template <class T>
 void launch_init_fields(const double *lc, const uint8_t *mask, const Geo &g, const SlotParams *sp,
                         const PropParams *pp, int nprops, int gaussian, double waist, double dx, double dy,
-                        C2<T> *F, hipStream_t st);
+                        C2<T> *F, bool x_slow, hipStream_t st);
 template <class T>
 void launch_pack_fields(const c64 *E, const Geo &g, const PropParams *pp, int nprops, int nq, C2<T> *F,
-                        hipStream_t st);
+                        bool x_slow, hipStream_t st);
 
 // slab boundary out = Pn Sh^nshift Pp in (cf_prev / cf_next may be null);
-// unshifted: every propagation's shift filter is the identity (pointwise kernel)
+// unshifted: every propagation's shift filter is the identity (pointwise kernel);
+// cf_prev / cf_next: coefficient tiles, or with x_slow the phase planes
 template <class T>
 void launch_boundary(const C2<T> *in, C2<T> *out, const C2<T> *cf_prev, const C2<T> *cf_next, const Geo &g,
-                     const PropParams *pp, int nprops, int nshift, bool unshifted, hipStream_t st);
+                     const PropParams *pp, int nprops, int nshift, bool unshifted, bool x_slow, hipStream_t st);
 // out = in + mu*A_y in (dir 1) or in + mu*A_x in (dir 0)
 template <class T>
 void launch_explicit(int dir, const C2<T> *in, C2<T> *out, const C2<T> *cf, const Geo &g, const PropParams *pp,
@@ -91,7 +116,7 @@ void launch_ysolve(int neumann, const C2<T> *src, C2<T> *dst, const C2<T> *accin
 // and the output Fresnel interface
 template <class T>
 void launch_output(const C2<T> *F, const double *lc, const uint8_t *mask, const Geo &g, const SlotParams *sp,
-                   const PropParams *pp, int nprops, int nq, c64 *E, hipStream_t st);
+                   const PropParams *pp, int nprops, int nq, c64 *E, bool x_slow, hipStream_t st);
 
 // output of a mesh of one plane: each full-grid point's entrance field (beam 0
 // uniform, 1 Gaussian, 2 the caller's fields already in E) through the output
@@ -109,7 +134,7 @@ void launch_bulk_entrance(const double *lc, const uint8_t *mask, const Geo &g, c
 // bulk[(((iwl*nq + iq)*2 + pol)*Nz + plane)*2 + comp][m] (complex128)
 template <class T>
 void launch_bulk_plane(const C2<T> *F, const Geo &g, const SlotParams *sp, const PropParams *pp, int nprops,
-                       int plane, int nq, c64 *bulk, hipStream_t st);
+                       int plane, int nq, c64 *bulk, bool x_slow, hipStream_t st);
 
 // screen filter: batched 2-D FFT of howmany planes (Ny x Nx) and the per-k
 // 2x2 transfer filter

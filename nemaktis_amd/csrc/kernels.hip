@@ -583,6 +583,147 @@ void launch_slab_coefs(const double *lc, const uint8_t *mask, const double *weig
 }
 
 // ---------------------------------------------------------------------------
+// Slab material of slabs iz0 .. for the solvers that generate the stencils
+// themselves (WalkRing; walk_kernels.hip) and the phase operators beside it.
+// Pointwise: a 16 x 16 tile per block, written through LDS so that both axis
+// orders are stored in runs of 16 points.
+// Bound by its own arithmetic and division chains at 64^2 and 128^2, by the
+// 55 MB it moves at 512^2: 19.7 us a slab there (the stencils, k_slab_coefs:
+// 34.8), 52.9 us at 1024^2 (139).
+// ---------------------------------------------------------------------------
+constexpr int kWalkTile = 16;
+
+template <class T>
+__global__ __launch_bounds__(256) void k_slab_material(const double *__restrict__ lc,
+                                                       const uint8_t *__restrict__ mask,
+                                                       const double *__restrict__ weights, Geo g,
+                                                       const SlotParams *__restrict__ sp, int iz0, int nslots,
+                                                       WalkRing<T> wr, int ring) {
+    constexpr int N2 = kWalkTile * kWalkTile, PITCH = N2 + 1;
+    __shared__ double mat[SM_COUNT * PITCH];
+    __shared__ C2<T> ph[3 * N2];
+    const int ntx = (g.Mx + kWalkTile - 1) / kWalkTile, nty = (g.My + kWalkTile - 1) / kWalkTile;
+    const int tile = xcd_tile(blockIdx.x, gridDim.x);
+    if (tile >= ntx * nty) return;
+    const int ix0 = (tile % ntx) * kWalkTile, iy0 = (tile / ntx) * kWalkTile;
+    const int slot = (int)blockIdx.y % nslots, iz = iz0 + (int)blockIdx.y / nslots;
+    const SlotParams s = sp[slot];
+    const int64_t N = g.Nfull;
+    const size_t NP = (size_t)g.NP;
+    const int t = threadIdx.x, lx = t % kWalkTile, ly = t / kWalkTile;
+    const int ix = ix0 + lx, iy = iy0 + ly;
+    if (ix < g.Mx && iy < g.My) {
+        const int64_t m = ix + (int64_t)g.Nx * iy;
+        VoxelData va, vb;
+        load_voxel(lc, mask, g.field_dim, m + N * iz, va);
+        load_voxel(lc, mask, g.field_dim, m + N * (iz + 1), vb);
+        double w = 0.5, wpz = 0.5;
+        if (weights) {
+            const int64_t v = m + N * iz;
+            w = weights[2 * v];
+            wpz = weights[2 * v + 1];
+        }
+        double a[12], b[12], f[SM_COUNT];
+        eps_of(va, g.field_dim, s, a);
+        eps_of(vb, g.field_dim, s, b);
+        slab_fields(a, b, f);
+#pragma unroll
+        for (int c = 0; c < SM_COUNT; c++) mat[c * PITCH + t] = f[c];
+        c64 pxx, pyy, pxy;
+        slab_phase(a, b, w, wpz, s, pxx, pyy, pxy);
+        ph[t] = cast2<T>(pxx);
+        ph[N2 + t] = cast2<T>(pyy);
+        ph[2 * N2 + t] = cast2<T>(pxy);
+    }
+    const size_t buf = (size_t)(iz % ring), pts = walk_points(g.Mx, g.My);
+    c64 *nat = wr.mat + buf * wr.mat_stride + (size_t)slot * pts * 5;
+    c64 *tr = nat + (size_t)nslots * pts * 5;
+    // the duplicate column and row, by threads of the last tiles (the corner by both: the same values)
+    const bool last_x = ix0 + kWalkTile >= g.Mx, last_y = iy0 + kWalkTile >= g.My;
+    if ((last_x && t <= kWalkTile) || (last_y && t >= 64 && t <= 64 + kWalkTile)) {
+        const bool col = t < 64;
+        const int k = col ? min(iy0 + t, g.My) : min(ix0 + t - 64, g.Mx);
+        const int gx = col ? g.Mx : k, gy = col ? k : g.My;       // the point's place
+        const int qx = gx == g.Mx ? 0 : gx, qy = gy == g.My ? 0 : gy;  // its periodic image
+        const int64_t m = qx + (int64_t)g.Nx * qy, d = gx + (int64_t)g.Nx * gy;
+        if (col ? gy < g.My ? t < kWalkTile : last_y : gx < g.Mx ? t < 64 + kWalkTile : last_x) {
+            double a[12], b[12], f[SM_COUNT];
+            eps_voxel(lc, mask, g.field_dim, m + N * iz, s, a);
+            eps_voxel(lc, mask, g.field_dim, m + N * (iz + 1), s, b);
+            slab_fields(a, b, f);
+            eps_voxel(lc, mask, g.field_dim, d + N * iz, s, a);
+            eps_voxel(lc, mask, g.field_dim, d + N * (iz + 1), s, b);
+            f[SM_EINV] = (1. / a[2] + 1. / b[2]) / 2;
+            c64 *o = nat + ((size_t)gy * (g.Mx + 1) + gx) * 5;
+            o[0] = c64{f[SM_KYY], f[SM_KXY]};
+            o[1] = c64{f[SM_KXX], f[SM_IYY]};
+            o[2] = c64{f[SM_IXY], f[SM_IXX]};
+            o[3] = c64{f[SM_EINV], f[SM_VX]};
+            o[4] = c64{f[SM_VY], 0.0};
+            o = tr + ((size_t)gx * (g.My + 1) + gy) * 5;
+            o[0] = c64{f[SM_KXX], f[SM_KXY]};
+            o[1] = c64{f[SM_KYY], f[SM_IXX]};
+            o[2] = c64{f[SM_IXY], f[SM_IYY]};
+            o[3] = c64{f[SM_EINV], f[SM_VY]};
+            o[4] = c64{f[SM_VX], 0.0};
+        }
+    }
+    __syncthreads();
+    const int nx = min(kWalkTile, g.Mx - ix0), ny = min(kWalkTile, g.My - iy0);
+#pragma unroll
+    for (int k = 0; k < 5; k++) {
+        const int e = t + k * 256, row = e / (5 * kWalkTile), off = e - row * (5 * kWalkTile);
+        const int pt = off / 5, c = off - pt * 5;
+        // members of value c for lines along y (nat) and along x (tr)
+        const int y0 = c == 0 ? SM_KYY : c == 1 ? SM_KXX : c == 2 ? SM_IXY : c == 3 ? SM_EINV : SM_VY;
+        const int y1 = c == 0 ? SM_KXY : c == 1 ? SM_IYY : c == 2 ? SM_IXX : SM_VX;
+        const int x0 = c == 0 ? SM_KXX : c == 1 ? SM_KYY : c == 2 ? SM_IXY : c == 3 ? SM_EINV : SM_VX;
+        const int x1 = c == 0 ? SM_KXY : c == 1 ? SM_IXX : c == 2 ? SM_IYY : SM_VY;
+        if (row < ny && pt < nx) {
+            const int at = row * kWalkTile + pt;
+            nat[((size_t)(iy0 + row) * (g.Mx + 1) + ix0) * 5 + off] =
+                c64{mat[y0 * PITCH + at], c == 4 ? 0.0 : mat[y1 * PITCH + at]};
+        }
+        if (row < nx && pt < ny) {
+            const int at = pt * kWalkTile + row;
+            tr[((size_t)(ix0 + row) * (g.My + 1) + iy0) * 5 + off] =
+                c64{mat[x0 * PITCH + at], c == 4 ? 0.0 : mat[x1 * PITCH + at]};
+        }
+    }
+    if (ly < nx && lx < ny) {  // x slow: consecutive threads along y
+        C2<T> *o = wr.phase + buf * wr.phase_stride + (size_t)slot * 3 * NP + (size_t)(ix0 + ly) * g.My + iy0 + lx;
+        const int at = lx * kWalkTile + ly;
+        o[0] = ph[at];
+        o[NP] = ph[N2 + at];
+        o[2 * NP] = ph[2 * N2 + at];
+    }
+}
+
+template <class T>
+void launch_slab_material(const double *lc, const uint8_t *mask, const double *weights, const Geo &g,
+                          const SlotParams *sp, int nslots, int iz0, int nz, const WalkRing<T> &wr, int ring,
+                          hipStream_t st) {
+    if (nz < 1 || nz > ring || (int64_t)nz * nslots > 65535)
+        throw std::runtime_error("slab material: bad slab batch");
+    const int64_t tiles = (int64_t)((g.Mx + kWalkTile - 1) / kWalkTile) * ((g.My + kWalkTile - 1) / kWalkTile);
+    const dim3 grid((unsigned)((tiles + 7) / 8 * 8), nslots * nz);
+    hipLaunchKernelGGL(k_slab_material<T>, grid, dim3(256), 0, st, lc, mask, weights, g, sp, iz0, nslots, wr, ring);
+    NMK_LAUNCH_CHECK();
+}
+
+// Point of the thread in a 16 x 16 tile of an nx x ny grid, 8 x 8 points per
+// wave: 128-byte runs in both axis orders of the state
+__device__ __forceinline__ bool tile_point(int nx, int ny, int &ix, int &iy) {
+    const int ntx = (nx + kWalkTile - 1) / kWalkTile, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    ix = (int)(blockIdx.x % ntx) * kWalkTile + (wave & 1) * 8 + (lane & 7);
+    iy = (int)(blockIdx.x / ntx) * kWalkTile + (wave >> 1) * 8 + (lane >> 3);
+    return ix < nx && iy < ny;
+}
+static inline unsigned tiles_for(int nx, int ny) {
+    return (unsigned)(((nx + kWalkTile - 1) / kWalkTile) * ((ny + kWalkTile - 1) / kWalkTile));
+}
+
+// ---------------------------------------------------------------------------
 // input beam (PhysicsLib/BeamProfile.cpp:17-39) + input Fresnel
 // (BeamPropagationLib/FresnelOperator.cpp:16-38), written to the march grid
 // ---------------------------------------------------------------------------
@@ -606,17 +747,25 @@ __device__ __forceinline__ void entrance_field(const double *__restrict__ lc, co
     b = -2 * n * nxy / det * E0 + 2 * n * (n + nxx) / det * E1;
 }
 
-template <class T>
+// XS: the state with x slow ([x][y], the order of the solvers that walk their lines), tile by tile
+template <class T, bool XS>
 __global__ __launch_bounds__(256) void k_init_fields(const double *__restrict__ lc, const uint8_t *__restrict__ mask,
                                                      Geo g, const SlotParams *__restrict__ sp,
                                                      const PropParams *__restrict__ pp, int gaussian, double waist,
                                                      double dx, double dy, C2<T> *__restrict__ F) {
-    const int64_t ip = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (ip >= g.NP) return;
+    int64_t ip = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    int ix, iy;
+    if (XS) {
+        if (!tile_point(g.Mx, g.My, ix, iy)) return;
+        ip = iy + (int64_t)g.My * ix;
+    } else {
+        if (ip >= g.NP) return;
+        ix = (int)(ip % g.Mx);
+        iy = (int)(ip / g.Mx);
+    }
     const int prop = blockIdx.y;
     const PropParams p = pp[prop];
     const SlotParams s = sp[p.slot];
-    const int ix = (int)(ip % g.Mx), iy = (int)(ip / g.Mx);
     double a, b;
     entrance_field(lc, mask, g, s, p, ix, iy, gaussian, waist, dx, dy, a, b);
     F[((int64_t)prop * 2 + 0) * g.NP + ip] = C2<T>{(T)a, (T)0};
@@ -663,28 +812,42 @@ void launch_bulk_entrance(const double *lc, const uint8_t *mask, const Geo &g, c
 template <class T>
 void launch_init_fields(const double *lc, const uint8_t *mask, const Geo &g, const SlotParams *sp,
                         const PropParams *pp, int nprops, int gaussian, double waist, double dx, double dy,
-                        C2<T> *F, hipStream_t st) {
-    hipLaunchKernelGGL(k_init_fields<T>, dim3(blocks_for(g.NP, 256), nprops), dim3(256), 0, st, lc, mask, g, sp, pp,
-                       gaussian, waist, dx, dy, F);
+                        C2<T> *F, bool x_slow, hipStream_t st) {
+    if (x_slow)
+        hipLaunchKernelGGL((k_init_fields<T, true>), dim3(tiles_for(g.Mx, g.My), nprops), dim3(256), 0, st, lc, mask,
+                           g, sp, pp, gaussian, waist, dx, dy, F);
+    else
+        hipLaunchKernelGGL((k_init_fields<T, false>), dim3(blocks_for(g.NP, 256), nprops), dim3(256), 0, st, lc, mask,
+                           g, sp, pp, gaussian, waist, dx, dy, F);
     NMK_LAUNCH_CHECK();
 }
 
-template <class T>
+template <class T, bool XS>
 __global__ __launch_bounds__(256) void k_pack_fields(const c64 *__restrict__ E, Geo g, C2<T> *__restrict__ F) {
-    const int64_t ip = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (ip >= g.NP) return;
+    int64_t ip = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    int ix, iy;
+    if (XS) {
+        if (!tile_point(g.Mx, g.My, ix, iy)) return;
+        ip = iy + (int64_t)g.My * ix;
+    } else {
+        if (ip >= g.NP) return;
+        ix = (int)(ip % g.Mx);
+        iy = (int)(ip / g.Mx);
+    }
     const int prop = blockIdx.y;
-    const int ix = (int)(ip % g.Mx), iy = (int)(ip / g.Mx);
     const int64_t m = ix + (int64_t)g.Nx * iy;
     for (int c = 0; c < 2; c++) F[((int64_t)prop * 2 + c) * g.NP + ip] = cast2<T>(E[((int64_t)prop * 2 + c) * g.Nfull + m]);
 }
 
 template <class T>
 void launch_pack_fields(const c64 *E, const Geo &g, const PropParams *pp, int nprops, int nq, C2<T> *F,
-                        hipStream_t st) {
+                        bool x_slow, hipStream_t st) {
     (void)pp;
     (void)nq;
-    hipLaunchKernelGGL(k_pack_fields<T>, dim3(blocks_for(g.NP, 256), nprops), dim3(256), 0, st, E, g, F);
+    if (x_slow)
+        hipLaunchKernelGGL((k_pack_fields<T, true>), dim3(tiles_for(g.Mx, g.My), nprops), dim3(256), 0, st, E, g, F);
+    else
+        hipLaunchKernelGGL((k_pack_fields<T, false>), dim3(blocks_for(g.NP, 256), nprops), dim3(256), 0, st, E, g, F);
     NMK_LAUNCH_CHECK();
 }
 
@@ -709,7 +872,27 @@ constexpr int kBTW = 64, kBTH = 8;
 // (TW+6) x (TH+6) input window is loaded once with the previous phase operator
 // applied, the x pass is done in place in LDS, then the y pass and the next
 // phase operator; wrapped window indices are computed once per block.
-template <class T>
+// XS: the state and the phase operators (three planes) are kept with x slow, so
+// that x and y trade places; g comes with its axes exchanged.
+template <class T, bool XS>
+struct PhaseOps {
+    const C2<T> *p;  // first value of the slot, or null
+    int Mx;
+    size_t stride;
+    __device__ __forceinline__ PhaseOps(const C2<T> *base, int slot, const Geo &g)
+        : p(!base ? nullptr
+            : XS  ? base + (size_t)slot * 3 * (size_t)g.NP
+                  : base + (size_t)slot * cf_slot_size(g.Mx, g.My) + CF_P * kCfTile),
+          Mx(g.Mx), stride(XS ? (size_t)g.NP : (size_t)kCfTile) {}
+    __device__ __forceinline__ void load(unsigned x, unsigned y, C2<T> (&o)[3]) const {
+        const C2<T> *q = p + (XS ? x + (unsigned)Mx * y : cf_point(x, y, Mx));
+        o[0] = q[0];
+        o[1] = q[stride];
+        o[2] = q[2 * stride];
+    }
+};
+
+template <class T, bool XS>
 __global__ __launch_bounds__(256) void k_boundary(const C2<T> *__restrict__ in, C2<T> *__restrict__ out,
                                                   const C2<T> *__restrict__ cf_prev, const C2<T> *__restrict__ cf_next,
                                                   Geo g, const PropParams *__restrict__ pp, int nshift) {
@@ -721,9 +904,11 @@ __global__ __launch_bounds__(256) void k_boundary(const C2<T> *__restrict__ in, 
     const PropParams p = pp[prop0];
     const size_t NP = (size_t)g.NP;
     const int x0 = blockIdx.x * kBTW, y0 = blockIdx.y * kBTH;
-    const double *wxs = nshift == 2 ? p.w2x : p.w1x, *wys = nshift == 2 ? p.w2y : p.w1y;
-    const int ox = g.px ? (nshift == 2 ? p.o2x : p.o1x) : 0;
-    const int oy = g.py ? (nshift == 2 ? p.o2y : p.o1y) : 0;
+    const double *wax = nshift == 2 ? p.w2x : p.w1x, *way = nshift == 2 ? p.w2y : p.w1y;
+    const int oax = nshift == 2 ? p.o2x : p.o1x, oay = nshift == 2 ? p.o2y : p.o1y;
+    const double *wxs = XS ? way : wax, *wys = XS ? wax : way;
+    const int ox = g.px ? (XS ? oay : oax) : 0;
+    const int oy = g.py ? (XS ? oax : oay) : 0;
     if ((int)threadIdx.x < WW) {
         const int i = x0 + ox + (int)threadIdx.x;
         colw[threadIdx.x] = g.px ? wrapm(i, g.Mx) : min(max(i, 0), g.Mx - 1);
@@ -733,7 +918,7 @@ __global__ __launch_bounds__(256) void k_boundary(const C2<T> *__restrict__ in, 
     }
     __syncthreads();
     const C *f = in + (size_t)prop0 * 2 * NP;  // planes: pol 0 (x, y), pol 1 (x, y)
-    const C *cp = cf_prev ? cf_prev + (size_t)p.slot * cf_slot_size(g.Mx, g.My) + CF_P * kCfTile : nullptr;
+    const PhaseOps<T, XS> cp(cf_prev, p.slot, g);
     // input window with the previous slab's phase operator applied: a
     // thread takes elements t, t + 256, ... and fetches all of them (fields
     // and phase operators) before it evaluates any
@@ -747,31 +932,21 @@ __global__ __launch_bounds__(256) void k_boundary(const C2<T> *__restrict__ in, 
             const unsigned q = colw[c] + (unsigned)g.Mx * roww[r];
 #pragma unroll
             for (int pl = 0; pl < 4; pl++) wf[k][pl] = f[pl * NP + q];
-            if (cp) {
-                const C *c3 = cp + cf_point(colw[c], roww[r], g.Mx);
-                wp[k][0] = c3[0];
-                wp[k][1] = c3[kCfTile];
-                wp[k][2] = c3[2 * kCfTile];
-            }
+            if (cp.p) cp.load(colw[c], roww[r], wp[k]);
         }
     }
     // the next slab's phase operators at the thread's output points t and
     // t + 256, fetched with the window
-    const C *cn = cf_next ? cf_next + (size_t)p.slot * cf_slot_size(g.Mx, g.My) + CF_P * kCfTile : nullptr;
+    const PhaseOps<T, XS> cn(cf_next, p.slot, g);
     static_assert(kBTH * kBTW == 2 * 256, "two output points per thread of a 256-thread block");
     C np3[2][3];
-    if (cn) {
+    if (cn.p) {
 #pragma unroll
         for (int k = 0; k < 2; k++) {
             const int e = threadIdx.x + k * 256;
             const int r = e / kBTW, c = e - r * kBTW;
             const int x = x0 + c, y = y0 + r;
-            if (x < g.Mx && y < g.My) {
-                const C *c3 = cn + cf_point(x, y, g.Mx);
-                np3[k][0] = c3[0];
-                np3[k][1] = c3[kCfTile];
-                np3[k][2] = c3[2 * kCfTile];
-            }
+            if (x < g.Mx && y < g.My) cn.load(x, y, np3[k]);
         }
     }
 #pragma unroll
@@ -780,7 +955,7 @@ __global__ __launch_bounds__(256) void k_boundary(const C2<T> *__restrict__ in, 
         if (e < WH * WW) {
             const int r = e / WW, c = e - r * WW;
             C a0 = wf[k][0], b0 = wf[k][1], a1 = wf[k][2], b1 = wf[k][3];
-            if (cp) {
+            if (cp.p) {
                 const C pxx = wp[k][0], pyy = wp[k][1], pxy = wp[k][2];
                 const C na0 = pxx * a0 + pxy * b0, nb0 = pxy * a0 + pyy * b0;
                 const C na1 = pxx * a1 + pxy * b1, nb1 = pxy * a1 + pyy * b1;
@@ -848,7 +1023,7 @@ __global__ __launch_bounds__(256) void k_boundary(const C2<T> *__restrict__ in, 
             v[pl] = a;
         }
         const unsigned q = x + (unsigned)g.Mx * y;
-        if (cn) {
+        if (cn.p) {
             const C pxx = np3[k][0], pyy = np3[k][1], pxy = np3[k][2];
 #pragma unroll
             for (int pol = 0; pol < 2; pol++) {
@@ -866,7 +1041,7 @@ __global__ __launch_bounds__(256) void k_boundary(const C2<T> *__restrict__ in, 
 
 // The same boundary when no propagation of the launch is shifted (normal
 // incidence: the Catmull-Rom filters are the identity), point by point
-template <class T>
+template <class T, bool XS>
 __global__ __launch_bounds__(256) void k_boundary_point(const C2<T> *__restrict__ in, C2<T> *__restrict__ out,
                                                         const C2<T> *__restrict__ cf_prev,
                                                         const C2<T> *__restrict__ cf_next, Geo g,
@@ -881,8 +1056,9 @@ __global__ __launch_bounds__(256) void k_boundary_point(const C2<T> *__restrict_
     C v[4] = {f[q], f[NP + q], f[2 * NP + q], f[3 * NP + q]};
     const unsigned qy = q / (unsigned)g.Mx, qx = q - qy * (unsigned)g.Mx;
     auto apply = [&](const C *cfx) {
-        const C *c3 = cfx + (size_t)slot * cf_slot_size(g.Mx, g.My) + CF_P * kCfTile + cf_point(qx, qy, g.Mx);
-        const C pxx = c3[0], pyy = c3[kCfTile], pxy = c3[2 * kCfTile];
+        C c3[3];
+        PhaseOps<T, XS>(cfx, slot, g).load(qx, qy, c3);
+        const C pxx = c3[0], pyy = c3[1], pxy = c3[2];
 #pragma unroll
         for (int pol = 0; pol < 2; pol++) {
             const C a = pxx * v[2 * pol] + pxy * v[2 * pol + 1], b = pxy * v[2 * pol] + pyy * v[2 * pol + 1];
@@ -901,14 +1077,21 @@ __global__ __launch_bounds__(256) void k_boundary_point(const C2<T> *__restrict_
 
 template <class T>
 void launch_boundary(const C2<T> *in, C2<T> *out, const C2<T> *cf_prev, const C2<T> *cf_next, const Geo &g,
-                     const PropParams *pp, int nprops, int nshift, bool unshifted, hipStream_t st) {
+                     const PropParams *pp, int nprops, int nshift, bool unshifted, bool x_slow, hipStream_t st) {
     if (nprops % 2) throw std::runtime_error("slab boundary: propagations come in polarisation pairs");
+    Geo e = g;
+    if (x_slow) {
+        std::swap(e.Mx, e.My);
+        std::swap(e.px, e.py);
+    }
     if (unshifted) {
         dim3 grid((unsigned)blocks_for(g.NP, 256), nprops / 2);
-        hipLaunchKernelGGL(k_boundary_point<T>, grid, dim3(256), 0, st, in, out, cf_prev, cf_next, g, pp);
+        if (x_slow) hipLaunchKernelGGL((k_boundary_point<T, true>), grid, dim3(256), 0, st, in, out, cf_prev, cf_next, e, pp);
+        else hipLaunchKernelGGL((k_boundary_point<T, false>), grid, dim3(256), 0, st, in, out, cf_prev, cf_next, e, pp);
     } else {
-        dim3 grid((g.Mx + kBTW - 1) / kBTW, (g.My + kBTH - 1) / kBTH, nprops / 2);
-        hipLaunchKernelGGL(k_boundary<T>, grid, dim3(256), 0, st, in, out, cf_prev, cf_next, g, pp, nshift);
+        dim3 grid((e.Mx + kBTW - 1) / kBTW, (e.My + kBTH - 1) / kBTH, nprops / 2);
+        if (x_slow) hipLaunchKernelGGL((k_boundary<T, true>), grid, dim3(256), 0, st, in, out, cf_prev, cf_next, e, pp, nshift);
+        else hipLaunchKernelGGL((k_boundary<T, false>), grid, dim3(256), 0, st, in, out, cf_prev, cf_next, e, pp, nshift);
     }
     NMK_LAUNCH_CHECK();
 }
@@ -2209,19 +2392,26 @@ void launch_ysolve(int neumann, const C2<T> *src, C2<T> *dst, const C2<T> *accin
 // shift phase, output Fresnel with each point's own eps at the last plane
 // (BeamPropagationLib/FresnelOperator.cpp:45-69)
 // ---------------------------------------------------------------------------
-template <class T>
+template <class T, bool XS>
 __global__ __launch_bounds__(256) void k_output(const C2<T> *__restrict__ F, const double *__restrict__ lc,
                                                 const uint8_t *__restrict__ mask, Geo g,
                                                 const SlotParams *__restrict__ sp, const PropParams *__restrict__ pp,
                                                 c64 *__restrict__ E) {
-    const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= g.Nfull) return;
+    int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    int ix, iy;
+    if (XS) {
+        if (!tile_point(g.Nx, g.Ny, ix, iy)) return;
+        m = ix + (int64_t)g.Nx * iy;
+    } else {
+        if (m >= g.Nfull) return;
+        ix = (int)(m % g.Nx);
+        iy = (int)(m / g.Nx);
+    }
     const int prop = blockIdx.y;
     const PropParams p = pp[prop];
     const SlotParams s = sp[p.slot];
-    const int ix = (int)(m % g.Nx), iy = (int)(m / g.Nx);
     const int jx = g.px ? ix % g.Mx : ix, jy = g.py ? iy % g.My : iy;
-    const int64_t ip = jx + (int64_t)g.Mx * jy;
+    const int64_t ip = XS ? jy + (int64_t)g.My * jx : jx + (int64_t)g.Mx * jy;
     const c64 ph = mk(p.ph_re, p.ph_im);
     const c64 a = ph * cast2<double>(F[((int64_t)prop * 2) * g.NP + ip]);
     const c64 b = ph * cast2<double>(F[((int64_t)prop * 2 + 1) * g.NP + ip]);
@@ -2236,9 +2426,14 @@ __global__ __launch_bounds__(256) void k_output(const C2<T> *__restrict__ F, con
 
 template <class T>
 void launch_output(const C2<T> *F, const double *lc, const uint8_t *mask, const Geo &g, const SlotParams *sp,
-                   const PropParams *pp, int nprops, int nq, c64 *E, hipStream_t st) {
+                   const PropParams *pp, int nprops, int nq, c64 *E, bool x_slow, hipStream_t st) {
     (void)nq;
-    hipLaunchKernelGGL(k_output<T>, dim3(blocks_for(g.Nfull, 256), nprops), dim3(256), 0, st, F, lc, mask, g, sp, pp, E);
+    if (x_slow)
+        hipLaunchKernelGGL((k_output<T, true>), dim3(tiles_for(g.Nx, g.Ny), nprops), dim3(256), 0, st, F, lc, mask, g,
+                           sp, pp, E);
+    else
+        hipLaunchKernelGGL((k_output<T, false>), dim3(blocks_for(g.Nfull, 256), nprops), dim3(256), 0, st, F, lc, mask,
+                           g, sp, pp, E);
     NMK_LAUNCH_CHECK();
 }
 
@@ -2294,19 +2489,26 @@ void launch_output_entrance(const double *lc, const uint8_t *mask, const Geo &g,
 // 2*plane shift half-steps applied so far, no interface;
 // bulk[(((iwl*nq + iq)*2 + pol)*Nz + plane)*2 + comp][m]
 // ---------------------------------------------------------------------------
-template <class T>
+template <class T, bool XS>
 __global__ __launch_bounds__(256) void k_bulk_plane(const C2<T> *__restrict__ F, Geo g,
                                                     const SlotParams *__restrict__ sp,
                                                     const PropParams *__restrict__ pp, int plane, int nq,
                                                     c64 *__restrict__ bulk) {
-    const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= g.Nfull) return;
+    int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    int ix, iy;
+    if (XS) {
+        if (!tile_point(g.Nx, g.Ny, ix, iy)) return;
+        m = ix + (int64_t)g.Nx * iy;
+    } else {
+        if (m >= g.Nfull) return;
+        ix = (int)(m % g.Nx);
+        iy = (int)(m / g.Nx);
+    }
     const int prop = blockIdx.y;
     const PropParams p = pp[prop];
     const int iwl = sp[p.slot].iwl;
-    const int ix = (int)(m % g.Nx), iy = (int)(m / g.Nx);
     const int jx = g.px ? ix % g.Mx : ix, jy = g.py ? iy % g.My : iy;
-    const int64_t ip = jx + (int64_t)g.Mx * jy;
+    const int64_t ip = XS ? jy + (int64_t)g.My * jx : jx + (int64_t)g.Mx * jy;
     double s, c;
     sincos(p.ph_half * 2.0 * plane, &s, &c);
     const c64 ph = mk(c, s);
@@ -2319,9 +2521,13 @@ __global__ __launch_bounds__(256) void k_bulk_plane(const C2<T> *__restrict__ F,
 
 template <class T>
 void launch_bulk_plane(const C2<T> *F, const Geo &g, const SlotParams *sp, const PropParams *pp, int nprops,
-                       int plane, int nq, c64 *bulk, hipStream_t st) {
-    hipLaunchKernelGGL(k_bulk_plane<T>, dim3(blocks_for(g.Nfull, 256), nprops), dim3(256), 0, st, F, g, sp, pp,
-                       plane, nq, bulk);
+                       int plane, int nq, c64 *bulk, bool x_slow, hipStream_t st) {
+    if (x_slow)
+        hipLaunchKernelGGL((k_bulk_plane<T, true>), dim3(tiles_for(g.Nx, g.Ny), nprops), dim3(256), 0, st, F, g, sp, pp,
+                           plane, nq, bulk);
+    else
+        hipLaunchKernelGGL((k_bulk_plane<T, false>), dim3(blocks_for(g.Nfull, 256), nprops), dim3(256), 0, st, F, g, sp,
+                           pp, plane, nq, bulk);
     NMK_LAUNCH_CHECK();
 }
 
@@ -2635,14 +2841,18 @@ void launch_filter(c64 *E, const Geo &g, const SlotParams *sp, int nslots, const
                                        const SlotParams *, int, int, int, C2<T> *, int64_t, C2<T> *, int64_t, int, \
                                        const LinePlan &, hipStream_t);                                              \
     template void launch_init_fields<T>(const double *, const uint8_t *, const Geo &, const SlotParams *,             \
-                                        const PropParams *, int, int, double, double, double, C2<T> *, hipStream_t);  \
-    template void launch_pack_fields<T>(const c64 *, const Geo &, const PropParams *, int, int, C2<T> *, hipStream_t); \
+                                        const PropParams *, int, int, double, double, double, C2<T> *, bool,        \
+                                        hipStream_t);                                                                \
+    template void launch_slab_material<T>(const double *, const uint8_t *, const double *, const Geo &,            \
+                                          const SlotParams *, int, int, int, const WalkRing<T> &, int, hipStream_t);  \
+    template void launch_pack_fields<T>(const c64 *, const Geo &, const PropParams *, int, int, C2<T> *, bool,      \
+                                        hipStream_t);                                                                \
     template void launch_boundary<T>(const C2<T> *, C2<T> *, const C2<T> *, const C2<T> *, const Geo &,             \
-                                     const PropParams *, int, int, bool, hipStream_t);                                      \
+                                     const PropParams *, int, int, bool, bool, hipStream_t);                                \
     template void launch_explicit<T>(int, const C2<T> *, C2<T> *, const C2<T> *, const Geo &, const PropParams *,    \
                                      int, hipStream_t);                                                               \
     template void launch_bulk_plane<T>(const C2<T> *, const Geo &, const SlotParams *, const PropParams *, int, \
-                                       int, int, c64 *, hipStream_t);                                           \
+                                       int, int, c64 *, bool, hipStream_t);                                     \
     template void launch_xsolve<T>(int, const C2<T> *, C2<T> *, const C2<T> *, C2<T> *, const C2<T> *,              \
                                    const C2<T> *, const Geo &, const PropParams *, int, const LinePlan &, int, int,  \
                                    int, int, hipStream_t);                                                            \
@@ -2651,7 +2861,7 @@ void launch_filter(c64 *E, const Geo &g, const SlotParams *sp, int nslots, const
     template size_t xsolve_lds_bytes<T>(const LinePlan &, int, int);                                                  \
     template size_t ysolve_lds_bytes<T>(const LinePlan &, int, int);                                                  \
     template void launch_output<T>(const C2<T> *, const double *, const uint8_t *, const Geo &, const SlotParams *,  \
-                                   const PropParams *, int, int, c64 *, hipStream_t);
+                                   const PropParams *, int, int, c64 *, bool, hipStream_t);
 NMK_INST(float)
 NMK_INST(double)
 

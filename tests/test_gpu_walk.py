@@ -1,0 +1,82 @@
+"""The walking line solvers (FP64, built-in shapes) against the solvers on
+stored stencils, which explicit launch shapes ask for and which are held to
+the CPU oracle: the same operators in another order of the same FP64
+operations, so the two differ by round-off.
+
+Tolerance: a slab applies about 100 rounded operations of a few ulp to a field
+value, with condition numbers of the line systems near 1 (diagonal 1 + O(mu)):
+1e-13 relative L2 over up to 6 slabs, taken ten times larger.
+"""
+import json
+
+import numpy as np
+import pytest
+
+from nemaktis_amd import bpm_backend, fields
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-12
+
+
+def _director(dims, seed):
+    """smooth periodic director with some noise in all components"""
+    Nx, Ny, Nz = dims
+    rng = np.random.default_rng(seed)
+    z, y, x = np.meshgrid(np.arange(Nz), np.arange(Ny) / max(1, Ny - 1), np.arange(Nx) / max(1, Nx - 1), indexing="ij")
+    n = np.stack([np.cos(2 * np.pi * x + 0.3 * z), np.sin(2 * np.pi * y - 0.2 * z),
+                  0.8 + 0.5 * np.cos(2 * np.pi * (x + y))], -1)
+    n += 0.2 * rng.standard_normal(n.shape)
+    return n / np.linalg.norm(n, axis=-1, keepdims=True)
+
+
+def _compare(dims, lc, s, mask=None, formula="", E_in=None, **kw):
+    print("[gpu case]", dims, flush=True)
+    js = json.dumps(s)
+    chunks = 64 if max(dims) <= 1025 else 128  # of at most 16 points
+    stored = {"x_chunks": chunks, "x_rows": 1, "y_chunks": chunks, "y_cols": 2}
+    a = bpm_backend.propagate(js, lc, mask_vals=mask, mask_formula=formula, E_in=E_in, **kw)
+    b = bpm_backend.propagate(js, lc, mask_vals=mask, mask_formula=formula, E_in=E_in, tuning=stored)
+    assert np.isfinite(a).all()
+    a, b = (v.reshape(v.shape[0], v.shape[1], 2, -1) for v in (a, b))
+    err = np.linalg.norm(a - b, axis=-1) / np.linalg.norm(b, axis=-1)
+    assert err.max() < TOL, err.max()
+
+
+# march lines of Nx - 1 and Ny - 1 points: the shortest (16) and longest (1024) with a launch shape and their outer
+# neighbours, every chunk length 2..8 with and without shorter chunks, each lines-per-block (2 above 512 points), last
+# strips of one line
+@pytest.mark.parametrize("Nx,Ny", [(17, 17), (18, 33), (16, 40), (40, 16), (34, 130), (129, 66), (200, 97), (258, 50),
+                                   (400, 19), (512, 18), (513, 20), (514, 21), (25, 769), (1024, 17), (18, 1025),
+                                   (1026, 17)])
+def test_line_lengths(Nx, Ny):
+    dims = (Nx, Ny, 4)
+    s = fields.make_settings(dims, (0.1, 0.13, 0.1), [0.6], wavevectors=((0.0, 0.0), (0.11, -0.07)), nhost="1.5")
+    _compare(dims, _director(dims, Nx + Ny), s)
+
+
+@pytest.mark.parametrize("nw", [0, 1, 2, 3])
+def test_neumann_depths_batched(nw):
+    """several wavelengths and pairs in one batch"""
+    dims = (67, 45, 6)
+    s = fields.make_settings(dims, (0.1, 0.1, 0.1), [0.5, 0.62], wavevectors=((0.0, 0.0), (0.1, 0.05), (-0.2, 0.1)),
+                             ne_imag="0.002", n_woodbury=nw)
+    _compare(dims, _director(dims, nw), s, wl_batch=0)
+
+
+@pytest.mark.parametrize("field_type", ["Director", "Q-tensor"])
+def test_masked_fields(field_type):
+    """formula weights at the droplet's surface, a host medium, caller fields"""
+    dims = (35, 50, 6)
+    lc, mask, formula = fields.droplet(*dims, (0.1, 0.1, 0.1), 1.2)
+    lc = np.asarray(lc).reshape(dims[2], dims[1], dims[0], 3)
+    if field_type != "Director":
+        x, y, z = (lc[..., i] for i in range(3))
+        lc = np.stack([x * x - 1 / 3, y * y - 1 / 3, z * z - 1 / 3, x * y, x * z, y * z], -1)
+    s = fields.make_settings(dims, (0.1, 0.1, 0.1), [0.55], wavevectors=((0.0, 0.0), (0.15, 0.1)), nhost="1.55",
+                             field_type=field_type, beam_profile="GaussianBeam(2.0)")
+    _compare(dims, lc, s, mask=mask, formula=formula)
+    rng = np.random.default_rng(7)
+    E = rng.standard_normal(fields.output_shape(s)) + 1j * rng.standard_normal(fields.output_shape(s))
+    s["Physics settings"]["Initial conditions"]["Beam profile"] = "None"
+    _compare(dims, lc, s, mask=mask, E_in=E)
