@@ -138,17 +138,17 @@ void launch_bulk_plane(const C2<T> *F, const Geo &g, const SlotParams *sp, const
 
 // screen filter: batched 2-D FFT of howmany planes (Ny x Nx) and the per-k
 // 2x2 transfer filter
-// radices of the stages, 4 bits each from the lowest (at most 16 stages)
-// direct: the length has a prime factor above 13 or does not fit the LDS
-// plans (more than 2048 points); its lines are transformed by a direct DFT
+// radices of the stages, 4 bits each from the lowest (at most 16 stages);
+// stages 0 and 1 may be 15, a prime above 13 given in big
+// direct: the length does not fit the LDS plans (more than 2048 points); its
+// lines are transformed by a direct DFT
 struct FftPlan {
     int n, nst;
     uint64_t radices;
+    int big[2];
     int direct;
 };
 FftPlan make_fft_plan(int n);
-// true when the length factors into the radices of the LDS plans (2..13)
-bool fft_supported(int n);
 // unnormalised DFT of lines of length n, sign -1 forward, +1 backward, with
 // the twiddle table tw[m] = exp(-2 pi i m / n): `lines` lines per plane, line
 // i of plane p starting at p*plane_size + i*line_stride, elements elem_stride
@@ -162,8 +162,6 @@ void launch_fft_rows(const c64 *src, c64 *dst, int Nx, int Ny, int planes, int s
                      const FftPlan &px, hipStream_t st);
 void launch_fft_cols(c64 *data, int Nx, int Ny, int planes, int sign, const c64 *tw_y, const FftPlan &py,
                      hipStream_t st);
-// adjacent columns per workgroup of the column pass (LDS 2*n*C complex128)
-int fft_cols_per_block(int n);
 void launch_filter(c64 *E, const Geo &g, const SlotParams *sp, int nslots, const double *qxy, int nq,
                    const double *iso_thick, const double *iso_index, int n_iso, double dx, double dy,
                    double z_foc, double NA, hipStream_t st);

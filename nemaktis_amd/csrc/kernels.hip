@@ -2536,39 +2536,39 @@ void launch_bulk_plane(const C2<T> *F, const Geo &g, const SlotParams *sp, const
 // columns per workgroup (rows of C consecutive values in HBM), both with the
 // Stockham stages of fft_device.h
 // ---------------------------------------------------------------------------
-bool fft_supported(int n) {
-    if (n < 1) return false;
-    int m = n;
-    for (int r : {8, 4, 2, 3, 5, 7, 11, 13})
-        while (m % r == 0) m /= r;
-    return m == 1;
-}
-
 FftPlan make_fft_plan(int n) {
     FftPlan pl{};
     pl.n = n;
     if (n < 1) throw std::runtime_error("FFT length must be positive");
-    if (!fft_supported(n) || n > 2048) {
+    if (n > 2048) {
         pl.direct = 1;
         return pl;
     }
     int m = n;
-    pl.nst = 0;
+    for (int r : {8, 4, 2, 3, 5, 7, 11, 13})
+        while (m % r == 0 && m > 1) m /= r;
+    // the primes above 13 first (at most two below 2048), where their stage
+    // has no or few twiddles
+    for (int r = 17; m > 1; r += 2)
+        while (m % r == 0) {
+            pl.radices |= (uint64_t)15 << (4 * pl.nst);
+            pl.big[pl.nst++] = r;
+            m /= r;
+        }
+    m = n;
+    for (int st = 0; st < pl.nst; st++) m /= pl.big[st];
     for (int r : {8, 4, 2, 3, 5, 7, 11, 13})
         while (m % r == 0 && m > 1) {
             if (pl.nst >= 16) throw std::runtime_error("FFT plan too deep");
             pl.radices |= (uint64_t)r << (4 * pl.nst++);
             m /= r;
         }
-    if (m != 1) throw std::runtime_error("FFT length " + std::to_string(n) + " has a prime factor above 13");
     return pl;
 }
 
-int fft_cols_per_block(int n) { return fft_lines_per_block(n, 8); }
-
 // rows: block b transforms lines C*b .. C*b+C-1 of the whole batch (each a
 // contiguous run of n values); src and dst may be the same buffer
-template <int C, bool ODD>
+template <int C, int MODE>
 __global__ __launch_bounds__(256) void k_fft_rows(const c64 *src, c64 *dst, int64_t nlines, FftPlan pl,
                                                   const c64 *__restrict__ tw, int sign) {
     extern __shared__ c64 fbuf[];
@@ -2580,12 +2580,12 @@ __global__ __launch_bounds__(256) void k_fft_rows(const c64 *src, c64 *dst, int6
     for (int t = threadIdx.x; t < C * n; t += blockDim.x) fbuf[t] = t < nl * n ? src[base + t] : mk(0.0, 0.0);
     for (int t = threadIdx.x; t < n; t += blockDim.x) stw[t] = tw[t];
     __syncthreads();
-    const c64 *res = fft_stages<C, true, ODD>(fbuf, fbuf + C * n, pl, stw, sign);
+    const c64 *res = fft_stages<C, true, MODE>(fbuf, fbuf + C * n, pl, stw, sign);
     for (int t = threadIdx.x; t < nl * n; t += blockDim.x) dst[base + t] = res[t];
 }
 
 // columns, in place: block (group g, plane) transforms columns C*g .. C*g+C-1
-template <int C, bool ODD>
+template <int C, int MODE>
 __global__ __launch_bounds__(256) void k_fft_cols(c64 *__restrict__ data, int Nx, int ngroups, int64_t nblocks,
                                                   FftPlan pl, const c64 *__restrict__ tw, int sign) {
     extern __shared__ c64 fbuf[];
@@ -2602,14 +2602,14 @@ __global__ __launch_bounds__(256) void k_fft_cols(c64 *__restrict__ data, int Nx
     }
     for (int t = threadIdx.x; t < n; t += blockDim.x) stw[t] = tw[t];
     __syncthreads();
-    const c64 *res = fft_stages<C, false, ODD>(fbuf, fbuf + n * C, pl, stw, sign);
+    const c64 *res = fft_stages<C, false, MODE>(fbuf, fbuf + n * C, pl, stw, sign);
     for (int t = threadIdx.x; t < n * C; t += blockDim.x) {
         const int i = t % C, y = t / C;
         if (x0 + i < Nx) plane[(int64_t)y * Nx + x0 + i] = res[t];
     }
 }
 
-// Direct DFT of lines (lengths the LDS plans do not take): a block holds C
+// Direct DFT of lines (above 2048 points): a block holds C
 // lines and the twiddle table in LDS; output k of a line is
 // sum_j x_j tw[(j k) mod n] (conjugated twiddles for sign +1), with the twiddle
 // index advanced by k per term (no products or divisions in the loop).
@@ -2668,22 +2668,20 @@ void launch_fft_rows(const c64 *src, c64 *dst, int Nx, int Ny, int planes, int s
         launch_dft_lines(src, dst, Nx, Ny, planes, (int64_t)Nx * Ny, Nx, 1, sign, tw_x, st);
         return;
     }
-    const int C = fft_lines_per_block(Nx, 16);
+    const int mode = fft_mode(px), C = fft_lines_per_block(Nx, 16, mode == FFT_ANY);
     const int64_t nlines = (int64_t)Ny * planes;
     const unsigned grid = (unsigned)((nlines + C - 1) / C);
     const size_t lds = fft_lds_bytes(Nx, C);
+    auto launch = [&](auto *kernel) {
+        allow_kernel_lds(reinterpret_cast<const void *>(kernel), lds);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds, st, src, dst, nlines, px, tw_x, sign);
+    };
     switch (C) {
-#define NMK_ROWS(CC)                                                                                          \
-    case CC:                                                                                                  \
-        if (fft_pow2(px)) {                                                                                   \
-            allow_kernel_lds(reinterpret_cast<const void *>(k_fft_rows<CC, false>), lds);                    \
-            hipLaunchKernelGGL((k_fft_rows<CC, false>), dim3(grid), dim3(256), lds, st, src, dst, nlines, px, \
-                               tw_x, sign);                                                                   \
-        } else {                                                                                              \
-            allow_kernel_lds(reinterpret_cast<const void *>(k_fft_rows<CC, true>), lds);                     \
-            hipLaunchKernelGGL((k_fft_rows<CC, true>), dim3(grid), dim3(256), lds, st, src, dst, nlines, px,  \
-                               tw_x, sign);                                                                   \
-        }                                                                                                     \
+#define NMK_ROWS(CC)                                              \
+    case CC:                                                      \
+        if (mode == FFT_POW2) launch(k_fft_rows<CC, FFT_POW2>);   \
+        else if (mode == FFT_SMALL) launch(k_fft_rows<CC, FFT_SMALL>); \
+        else launch(k_fft_rows<CC, FFT_ANY>);                     \
         break;
         NMK_ROWS(16)
         NMK_ROWS(8)
@@ -2702,23 +2700,21 @@ void launch_fft_cols(c64 *data, int Nx, int Ny, int planes, int sign, const c64 
         launch_dft_lines(data, data, Ny, Nx, planes, (int64_t)Nx * Ny, 1, Nx, sign, tw_y, st);
         return;
     }
-    const int C = fft_cols_per_block(Ny);
+    const int mode = fft_mode(py), C = fft_lines_per_block(Ny, 8, mode == FFT_ANY);
     const int ngroups = (Nx + C - 1) / C;
     const int64_t nblocks = (int64_t)ngroups * planes;
     const unsigned grid = (unsigned)((nblocks + 7) / 8 * 8);
     const size_t lds = fft_lds_bytes(Ny, C);
+    auto launch = [&](auto *kernel) {
+        allow_kernel_lds(reinterpret_cast<const void *>(kernel), lds);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds, st, data, Nx, ngroups, nblocks, py, tw_y, sign);
+    };
     switch (C) {
-#define NMK_COLS(CC)                                                                                          \
-    case CC:                                                                                                  \
-        if (fft_pow2(py)) {                                                                                   \
-            allow_kernel_lds(reinterpret_cast<const void *>(k_fft_cols<CC, false>), lds);                    \
-            hipLaunchKernelGGL((k_fft_cols<CC, false>), dim3(grid), dim3(256), lds, st, data, Nx, ngroups,    \
-                               nblocks, py, tw_y, sign);                                                      \
-        } else {                                                                                              \
-            allow_kernel_lds(reinterpret_cast<const void *>(k_fft_cols<CC, true>), lds);                     \
-            hipLaunchKernelGGL((k_fft_cols<CC, true>), dim3(grid), dim3(256), lds, st, data, Nx, ngroups,     \
-                               nblocks, py, tw_y, sign);                                                      \
-        }                                                                                                     \
+#define NMK_COLS(CC)                                              \
+    case CC:                                                      \
+        if (mode == FFT_POW2) launch(k_fft_cols<CC, FFT_POW2>);   \
+        else if (mode == FFT_SMALL) launch(k_fft_cols<CC, FFT_SMALL>); \
+        else launch(k_fft_cols<CC, FFT_ANY>);                     \
         break;
         NMK_COLS(8)
         NMK_COLS(4)

@@ -77,9 +77,14 @@ void launch_view_filter(c64 *filt, int Nx, int Ny, double dx, double dy, const V
 // columns, product with the filter plane of their (wavelength, wavevector),
 // backward transform.  Work items run component-fastest and each XCD takes a
 // contiguous range, so the four components reading one filter tile share L2.
+// With any radix a third wave per SIMD is worth holding registers back for
+// (161^2, 532 planes: 379 -> 278 us).
 // ---------------------------------------------------------------------------
-template <int C, bool ODD, int NT = 256>
-__global__ __launch_bounds__(NT) void k_view_columns(c64 *__restrict__ data, const c64 *__restrict__ filt, int Nx,
+// most values a block holds
+constexpr int view_block_values(int mode, int C) { return mode == FFT_ANY && C < 8 ? 4096 : 2048; }
+
+template <int C, int MODE, int NT = 256>
+__global__ __launch_bounds__(NT, MODE == FFT_ANY ? 3 : 1) void k_view_columns(c64 *__restrict__ data, const c64 *__restrict__ filt, int Nx,
                                                       int ngroups, int64_t nitems, FftPlan pl,
                                                       const c64 *__restrict__ tw) {
     extern __shared__ c64 fbuf[];
@@ -95,8 +100,8 @@ __global__ __launch_bounds__(NT) void k_view_columns(c64 *__restrict__ data, con
     const c64 *fp = filt + lq * N;
     const int x0 = g * C;
     c64 *stw = fbuf + 2 * C * n;
-    // the filter values this thread multiplies, loaded with the fields (n * C <= 2048)
-    constexpr int kPer = 2048 / NT;
+    // the filter values this thread multiplies, loaded with the fields
+    constexpr int kPer = view_block_values(MODE, C) / NT;
     c64 fr[kPer];
 #pragma unroll
     for (int e = 0; e < kPer; e++) {
@@ -110,14 +115,14 @@ __global__ __launch_bounds__(NT) void k_view_columns(c64 *__restrict__ data, con
     }
     for (int t = threadIdx.x; t < n; t += blockDim.x) stw[t] = tw[t];
     __syncthreads();
-    c64 *a = fft_stages<C, false, ODD>(fbuf, fbuf + n * C, pl, stw, -1);
+    c64 *a = fft_stages<C, false, MODE>(fbuf, fbuf + n * C, pl, stw, -1);
 #pragma unroll
     for (int e = 0; e < kPer; e++) {
         const int t = threadIdx.x + e * NT;
         if (t < n * C) a[t] = a[t] * fr[e];
     }
     __syncthreads();
-    const c64 *r = fft_stages<C, false, ODD>(a, a == fbuf ? fbuf + n * C : fbuf, pl, stw, +1);
+    const c64 *r = fft_stages<C, false, MODE>(a, a == fbuf ? fbuf + n * C : fbuf, pl, stw, +1);
     for (int t = threadIdx.x; t < n * C; t += blockDim.x) {
         const int i = t % C, y = t / C;
         if (x0 + i < Nx) plane[(int64_t)y * Nx + x0 + i] = r[t];
@@ -147,32 +152,29 @@ void launch_view_columns(c64 *data, const c64 *filt, int Nx, int Ny, int nlq, co
     }
     // power-of-two columns of at most 256 points: eight adjacent columns per
     // block of 512 threads, so that a row of the block is a whole 128-byte line
-    const bool wide = fft_pow2(py) && 8 * Ny <= 2048 && Nx >= 8;
-    const int C = wide ? 8 : fft_cols_per_block(Ny);
-    if (Ny * C > 8 * 256) throw std::runtime_error("refocus columns: more than 2048 values per block");
+    const int mode = fft_mode(py);
+    const bool wide = mode == FFT_POW2 && 8 * Ny <= 2048 && Nx >= 8;
+    const int C = wide ? 8 : fft_lines_per_block(Ny, 8, mode == FFT_ANY);
+    if (Ny * C > view_block_values(mode, C)) throw std::runtime_error("refocus columns: too many values per block");
     const int ngroups = (Nx + C - 1) / C;
     const int64_t nitems = (int64_t)ngroups * nlq * 4;
     const unsigned grid = (unsigned)((nitems + 7) / 8 * 8);
     const size_t lds = fft_lds_bytes(Ny, C);
-    if (wide) {
-        allow_kernel_lds(reinterpret_cast<const void *>(k_view_columns<8, false, 512>), lds);
-        hipLaunchKernelGGL((k_view_columns<8, false, 512>), dim3(grid), dim3(512), lds, st, data, filt, Nx, ngroups,
-                           nitems, py, tw_y);
+    auto launch = [&](auto *kernel, int threads) {
+        allow_kernel_lds(reinterpret_cast<const void *>(kernel), lds);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds, st, data, filt, Nx, ngroups, nitems, py, tw_y);
         NMK_VIEW_LAUNCH_CHECK();
+    };
+    if (wide) {
+        launch(k_view_columns<8, FFT_POW2, 512>, 512);
         return;
     }
     switch (C) {
-#define NMK_VCOLS(CC)                                                                                         \
-    case CC:                                                                                                  \
-        if (fft_pow2(py)) {                                                                                   \
-            allow_kernel_lds(reinterpret_cast<const void *>(k_view_columns<CC, false>), lds);                \
-            hipLaunchKernelGGL((k_view_columns<CC, false>), dim3(grid), dim3(256), lds, st, data, filt, Nx,   \
-                               ngroups, nitems, py, tw_y);                                                    \
-        } else {                                                                                              \
-            allow_kernel_lds(reinterpret_cast<const void *>(k_view_columns<CC, true>), lds);                 \
-            hipLaunchKernelGGL((k_view_columns<CC, true>), dim3(grid), dim3(256), lds, st, data, filt, Nx,    \
-                               ngroups, nitems, py, tw_y);                                                    \
-        }                                                                                                     \
+#define NMK_VCOLS(CC)                                                      \
+    case CC:                                                               \
+        if (mode == FFT_POW2) launch(k_view_columns<CC, FFT_POW2>, 256);   \
+        else if (mode == FFT_SMALL) launch(k_view_columns<CC, FFT_SMALL>, 256); \
+        else launch(k_view_columns<CC, FFT_ANY>, 256);                     \
         break;
         NMK_VCOLS(8)
         NMK_VCOLS(4)
@@ -181,7 +183,6 @@ void launch_view_columns(c64 *data, const c64 *filt, int Nx, int Ny, int nlq, co
 #undef NMK_VCOLS
     default: throw std::runtime_error("refocus columns: bad block shape");
     }
-    NMK_VIEW_LAUNCH_CHECK();
 }
 
 // ---------------------------------------------------------------------------
