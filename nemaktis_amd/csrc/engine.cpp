@@ -143,19 +143,30 @@ int pow2_at_least(int v) {
 }
 
 // Launch shape of the walking solvers for lines of M points, Mt of them per
-// component and propagation: chunks of at most 8 points (16 spill), as many as
-// bring the threads of a launch to 128 K, up to 64; as many lines per block as
-// fit 512 threads of both components, up to 8.  W = 0: no shape (lines over
-// 1024 or under 16 points).
+// component and propagation: P chunks of a line and W lines a block, at most
+// 512 threads of both components, whole waves of one component; chunks of at
+// most 8 points (16 spill).  W = 0: no shape (lines over 1024 or under 16
+// points).
+//
+// A block is alone on its CU, so up to 256 blocks a launch takes as long as
+// one of them: as few lines a block as keep to that, and chunks of at most 6
+// points if the launch still fits (us a slab at one pair: 64^2 54 at 4 lines,
+// 61 at 8, 76 at 16; 161^2 74 / 76 / 99 at 2 / 4 / 8, and 78 with chunks of 3
+// for 5; 256^2 100 with chunks of 4, 105 with 8; 512^2 184 at 4 lines, 236 in
+// the two rounds of 2).  Beyond, the blocks' own work counts: long chunks, whose two extra
+// rows weigh less, and many lines, whose two extra columns do (128^2 x 294
+// propagations 1270 us at 16 lines, 1504 at 8, 2161 at 4).
 WalkShape walk_shape(int M, int Mt, int nprops) {
     WalkShape sh{};
     if (M > 1024) return sh;
-    const int64_t lines = (int64_t)Mt * 2 * nprops;
-    int par = 1;
-    while (par < 64 && (int64_t)par * lines < 131072) par *= 2;
-    sh.lp = make_line_plan(M, std::max(16, std::max(pow2_at_least((M + 7) / 8), par)));
-    for (sh.W = 8; sh.W > 1; sh.W /= 2)
-        if (2 * sh.W * sh.lp.P <= 512 && sh.W * sh.lp.P % 64 == 0) return sh;
+    auto fits = [&](int W) { return 2 * W * sh.lp.P <= 512 && W * sh.lp.P % 64 == 0; };
+    for (int most : {6, 8}) {
+        sh.lp = make_line_plan(M, std::max(16, pow2_at_least((M + most - 1) / most)));
+        for (sh.W = 2; sh.W <= 16; sh.W *= 2)
+            if (fits(sh.W) && (int64_t)((Mt + sh.W - 1) / sh.W) * nprops <= 256) return sh;
+    }
+    for (sh.W = 16; sh.W > 1; sh.W /= 2)
+        if (fits(sh.W)) return sh;
     sh.W = 0;
     return sh;
 }
@@ -816,11 +827,13 @@ private:
     //
     // FP64 marches at the built-in shapes take the walking solvers wherever
     // they have a shape (both axes periodic, march lines of 16 to 1024
-    // points): 25.1 -> 17.2 ms for 512^2 x 100 at one propagation pair, 267.5
-    // -> 171.5 ms for 1024^2 x 200, 22.6 -> 21.1 ms for a 128^2 x 40 call at
-    // 7 pairs, even at 64^2 (1.25 ms).  Explicit shapes are shapes of the
-    // solvers on stored stencils; FP32 stays there too, where the stencils are
-    // half the bytes and the walk's FP64 arithmetic is not.
+    // points): 25.1 -> 17.5 ms for 512^2 x 100 at one propagation pair, 267.5
+    // -> 171.5 ms for 1024^2 x 200, a slab of 96 x 80 at 70 pairs 371 -> 337
+    // us, of 256^2 at 147 pairs 6.2 -> 5.5 ms.  Explicit shapes are shapes of the
+    // solvers on stored stencils.  FP32 stays there too: its stencils are half
+    // the bytes and shared by the propagations of a wavelength, where the walk
+    // generates them for each (256^2 at 147 pairs 771-789 us a launch against
+    // 416-567, 512^2 at one pair 24 against 18-24).
     void set_tuning(const Tuning &asked) {
         const bool builtin = asked.x_chunks <= 0;
         WalkShape wx{}, wy{};

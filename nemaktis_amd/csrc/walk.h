@@ -13,7 +13,7 @@ struct WalkMaterial {
     const c64 *nat, *tr;
 };
 
-// launch shape of one axis: chunks of a line, lines per block (8, 4 or 2)
+// launch shape of one axis: chunks of a line, lines per block (16, 8, 4 or 2)
 struct WalkShape {
     LinePlan lp;
     int W;

@@ -22,10 +22,10 @@
 // row of the two) and 69-86 MB of traffic a launch; at 64^2 the chain of steps
 // and cyclic reductions.  Device time per launch, MI355X, against the solvers
 // on stored stencils (x / y lines): 512^2 x 1 pair 22-23 us (29-36 / 34-36),
-// 1024^2 120-125 us (130-156 / 225-238), 128^2 x 7 pairs 14.3 us (14 / 18-19),
-// 64^2 8.8 us (8 / 10); the slab's material 20 us instead of 35 us of stencils
-// at 512^2.  A whole 512^2 x 100 propagation 25.1 -> 17.2 ms, 1024^2 x 200
-// 267.5 -> 171.5 ms.
+// 1024^2 120-125 us (130-156 / 225-238).  Per slab, whole march: 64^2 54 us
+// (68), 161^2 74 us (96), 128^2 x 7 pairs 109 us (120), x 147 pairs 1.27 ms
+// (1.46), 256^2 x 147 pairs 5.5 ms (6.2).  A whole 512^2 x 100 propagation
+// 25.1 -> 17.5 ms, 1024^2 x 200 267.5 -> 171.5 ms.
 //
 // Lanes of a wave lie across the lines (consecutive in memory) and chunks of
 // them: the state is kept with the line axis slow, [l][t] for lines along l.
@@ -475,7 +475,7 @@ __global__ __launch_bounds__(512) void k_walk(const c64 *__restrict__ src, c64 *
     // the rows; later the reduced systems, then the result
     __shared__ c64 rows0[R::buffer], rows1[R::buffer], rows2[R::NB > 2 ? R::buffer : 1];
     auto rows = [&](int k) { return k == 0 ? rows0 : k == 1 ? rows1 : rows2; };
-    constexpr int lw = W == 8 ? 3 : W == 4 ? 2 : W == 2 ? 1 : 0;
+    constexpr int lw = W == 16 ? 4 : W == 8 ? 3 : W == 4 ? 2 : 1;
     const int P = lp.P, TW = P * W, NT = 2 * TW;
     const int Ml = axis == 0 ? g.Mx : g.My, Mt = axis == 0 ? g.My : g.Mx;
     const int nstrip = (Mt + W - 1) / W;
@@ -674,6 +674,7 @@ void launch_walk(int axis, int neumann, const c64 *src, c64 *dst, const c64 *acc
         else walk_dispatch<WW, 0>(sh, grid, src, dst, accin, acc, wm, axis, flip, g, sp, pp, nprops, per_slot, st);         \
         return;                                                                                                         \
     }
+    NMK_WALK(16)
     NMK_WALK(8)
     NMK_WALK(4)
     NMK_WALK(2)
