@@ -933,14 +933,17 @@ private:
 // y strips are as wide as the block allows up to one coefficient tile.
 Tuning default_tuning(int precision, int Mx, int My, int nprops) {
     Tuning t;
-    // a batch of at least 131072 lines per launch fills the device without
-    // splitting lines finely: 8-point chunks (at most 64 per line, so the
-    // reduced systems stay in one wave) and the register-lean solvers (more
-    // blocks in flight); measured on the 256^2 x 294-propagation FP32 sweep,
-    // 270.4 -> 261.5 ms per graph replay
-    const bool big = std::max(Mx, My) <= 512 && (int64_t)std::max(Mx, My) * 2 * std::max(2, nprops) >= 131072;
-    const int lcap = precision == 32 && !big ? 16 : 8;
-    if (big && precision == 32) t.lean = 1;
+    // FP32 batches on lines of up to 512 points: 8-point chunks (at most 64 per
+    // line, so the reduced systems stay in one wave) and the register-lean
+    // solvers (more blocks in flight), us a slab in graph replays before and
+    // after: 256^2 at 147 pairs 3418 -> 3309, 301 x 203 at 21 pairs 631 -> 554,
+    // 400 x 300 at 28 pairs 1639 -> 1503, 128^2 at 14 pairs 161 -> 131, 512^2 at
+    // 2 pairs 352 -> 314; a lone pair gains up to 400 points (256^2 109 -> 106)
+    // and loses at 512 (188 -> 191)
+    const int longest = std::max(Mx, My);
+    const bool lean = precision == 32 && longest <= 512 && (nprops > 2 || longest <= 400);
+    const int lcap = precision == 32 && !lean ? 16 : 8;
+    if (lean) t.lean = 1;
     auto chunks = [&](int M, int other) {
         const int64_t lines = (int64_t)std::max(1, other) * 2 * std::max(2, nprops);
         int par = 1;
@@ -974,6 +977,10 @@ Tuning default_tuning(int precision, int Mx, int My, int nprops) {
     t.y_cols = std::max(1, std::min(kCfTw, 512 / t.y_chunks));
     if (My > 3)
         while (t.y_cols > 1 && (t.y_chunks * t.y_cols > 512 || ylds(t.y_chunks, t.y_cols) > budget)) t.y_cols /= 2;
+    // at most 64 blocks leave most CUs idle: half-width strips instead (a lone
+    // pair on 256^2 106 -> 100 us a slab, 128^2 74 -> 72; with 76 blocks, 301 x
+    // 203, 112 -> 118)
+    while (precision == 32 && t.y_cols > 4 && (int64_t)((Mx + t.y_cols - 1) / t.y_cols) * nprops <= 64) t.y_cols /= 2;
     // slab coefficients on the march stream: as fast or faster than the second
     // stream on every measured batch (up to 12% on small ones, in graph replay)
     t.coef_serial = 1;
