@@ -70,6 +70,22 @@ def algorithmic_bytes(fam, c, nprops, nslots, NP, Nfull, fd, nw):
     return None
 
 
+# the FP64 march at the built-in shapes (mesh axes of 17 to 1025 points): solvers that generate their stencils
+KERNELS_WALK = {"solve_x": "k_walk", "solve_y": "k_walk", "boundary": "k_boundary", "coefs": "k_slab_material"}
+
+
+def walk_bytes(fam, nprops, nslots, NP, Nfull, fd, nw):
+    """algorithmic_bytes of the march that KERNELS_WALK names: the line solves
+    read 5 material values of 16 bytes a point and slot, which the coefficient
+    kernel writes in both axis orders beside 3 phase-operator planes."""
+    if fam in ("solve_x", "solve_y"):
+        planes = 4 + sum(2 + (2 if i > 0 else 0) + 2 + (2 if i + 1 < nw else 0) for i in range(nw))
+        return (planes * nprops * 16 / (1 + nw) + 80 * nslots) * NP
+    if fam == "coefs":
+        return 2 * fd * 8 * Nfull + (160 + 48) * nslots * NP
+    return algorithmic_bytes(fam, 16, nprops, nslots, NP, Nfull, fd, nw)
+
+
 TRAFFIC_FILE_IMAGING = os.path.join(ROOT, "profiles", "hbm_traffic_imaging_droplet256.txt")
 
 
@@ -480,11 +496,16 @@ def roofline_of(js, lc, n_E, precision, wl_batch, steps, Nx, Ny, nprops, nq, fd,
     algo = per_update * units
     achieved = algo / (avg_ms * 1e-3) / 1e9
     c = 8 if precision == 32 else 16
-    local = algorithmic_bytes(dom, c, nprops, nprops // (2 * nq), (Nx - 1) * (Ny - 1), Nx * Ny, fd, nw)
-    tag = "fp32" if precision == 32 else "fp64"
-    traffic, traffic_src = measured_traffic(KERNELS.get(dom, dom), os.path.join(ROOT, "profiles",
-                                                                              "hbm_traffic_random512_%s.txt" % tag))
-    return {"bound": "hbm", "kernel": KERNELS.get(dom, dom), "family": dom, "precision": precision,
+    walk = precision == 64 and tuning is None and 17 <= min(Nx, Ny) and max(Nx, Ny) <= 1025
+    if walk:
+        local = walk_bytes(dom, nprops, nprops // (2 * nq), (Nx - 1) * (Ny - 1), Nx * Ny, fd, nw)
+    else:
+        local = algorithmic_bytes(dom, c, nprops, nprops // (2 * nq), (Nx - 1) * (Ny - 1), Nx * Ny, fd, nw)
+    kernel = (KERNELS_WALK if walk else KERNELS).get(dom, dom)
+    tag = "fp32" if precision == 32 else "fp64_walk" if walk else "fp64"
+    traffic, traffic_src = measured_traffic(kernel, os.path.join(ROOT, "profiles",
+                                                                 "hbm_traffic_random512_%s.txt" % tag))
+    return {"bound": "hbm", "kernel": kernel, "family": dom, "precision": precision,
             "avg_launch_ms": avg_ms, "launches": fam_n[dom], "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": traffic,
             "traffic_source": traffic_src,

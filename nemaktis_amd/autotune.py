@@ -107,7 +107,7 @@ def _save_cache(c):
 
 
 def cache_key(precision, Nx, Ny, nprops, use_graph=True):
-    return "gfx950|solver-v13|%d|%dx%d|%d|%s" % (precision, Nx, Ny, nprops, "graph" if use_graph else "eager")
+    return "gfx950|solver-v14|%d|%dx%d|%d|%s" % (precision, Nx, Ny, nprops, "graph" if use_graph else "eager")
 
 
 def _time(ctx, tuning, reps):
@@ -126,7 +126,8 @@ def _time(ctx, tuning, reps):
 
 
 def tune(settings, lc_vals, precision=32, wl_batch=0, depth=9, reps=3, use_cache=True, log=None, use_graph=True):
-    """Returns the best tuning dict for this job's transverse mesh, measured
+    """Returns the best tuning dict for this job's transverse mesh (None: the
+    built-in shapes), measured
     on a `depth`-plane copy of it (graph replay or eager launches, as the job
     will run), plus the timing table."""
     ic = settings["Physics settings"]["Initial conditions"]
@@ -155,6 +156,12 @@ def tune(settings, lc_vals, precision=32, wl_batch=0, depth=9, reps=3, use_cache
     ctx = bpm_backend.Context(js, lc, n_E, precision=precision, wl_batch=wl_batch, use_graph=use_graph, tuning=best)
     try:
         best, best_ms, table, t0 = _search(ctx, best, xs, ys, Mx, My, precision, reps)
+        # the built-in shapes, which in FP64 march with other solvers than explicit ones ask for
+        # (512^2, one pair: 17.5 ms against 25 ms for the best explicit shape)
+        ms = _time(ctx, None, reps)
+        table.append((None, ms))
+        if ms <= best_ms:
+            best, best_ms = None, ms
     finally:
         ctx.close()
     if log:
