@@ -80,3 +80,22 @@ def test_masked_fields(field_type):
     E = rng.standard_normal(fields.output_shape(s)) + 1j * rng.standard_normal(fields.output_shape(s))
     s["Physics settings"]["Initial conditions"]["Beam profile"] = "None"
     _compare(dims, lc, s, mask=mask, E_in=E)
+
+
+@pytest.mark.parametrize("use_graph", [False, True])
+def test_retuning_to_stored_stencils_and_back(use_graph):
+    """a resident job whose solvers change gives each route's own result"""
+    dims = (40, 36, 5)
+    s = fields.make_settings(dims, (0.1, 0.1, 0.1), [0.6], wavevectors=((0.0, 0.0), (0.1, 0.05)))
+    lc = _director(dims, 11)
+    shape = fields.output_shape(s)
+    out = []
+    with bpm_backend.Context(json.dumps(s), lc, int(np.prod(shape)), precision=64, use_graph=use_graph) as ctx:
+        for tuning in (None, {"x_chunks": 16, "x_rows": 2, "y_chunks": 16, "y_cols": 8}, None):
+            if out:
+                ctx.set_tuning(tuning)
+            for _ in range(2):
+                ctx.propagate()
+            out.append(ctx.download(np.empty(shape, np.complex128)))
+    assert np.array_equal(out[0], out[2])
+    assert np.linalg.norm(out[0] - out[1]) < TOL * np.linalg.norm(out[1])
