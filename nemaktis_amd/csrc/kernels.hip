@@ -1512,102 +1512,96 @@ __device__ __forceinline__ C2<T> shfl_c(C2<T> v, int lane) {
 // The cyclic system of one line held by P <= 64 consecutive lanes of one wave
 // (lane lb + p holds interface row p): parallel cyclic reduction through lane
 // permutes, without LDS or barriers; returns xi_p.  Every lane of the wave
-// calls it (lanes of inactive lines compute unused values).  The rows are kept
-// normalised, x_p + a x_{p-s} + c x_{p+s} = d: three values to fetch from each
-// neighbour and one reciprocal a stage, where A, B, C, D take four and two
-// (with interface_solve: 512^2 FP32 at one pair 16.91 -> 16.74 ms a
-// propagation, 256^2 at 147 pairs y 545 -> 537 us a launch, 301 x 203 at 21
-// pairs 30.0 -> 29.5 ms; the solvers stay bound by the vector memory path).
+// calls it (lanes of inactive lines compute unused values).
 template <class T>
 __device__ __forceinline__ C2<T> wave_pcr(C2<T> A, C2<T> B, C2<T> Cc, C2<T> D, int P, int p, int lb) {
     using C = C2<T>;
-    const C one{(T)1, (T)0}, ib = crcp(B);
-    C a = A * ib, c = Cc * ib, d = D * ib;
     for (int st = 1; 2 * st < P; st <<= 1) {
         const int lm = lb + ((p - st) & (P - 1)), lq = lb + ((p + st) & (P - 1));
-        const C am = shfl_c(a, lm), cm = shfl_c(c, lm), dm = shfl_c(d, lm);
-        const C aq = shfl_c(a, lq), cq = shfl_c(c, lq), dq = shfl_c(d, lq);
-        const C iv = crcp(one - a * cm - c * aq);
-        d = (d - a * dm - c * dq) * iv;
-        a = -(a * am) * iv;
-        c = -(c * cq) * iv;
+        const C Am = shfl_c(A, lm), Bm = shfl_c(B, lm), Cm = shfl_c(Cc, lm), Dm = shfl_c(D, lm);
+        const C Aq = shfl_c(A, lq), Bq = shfl_c(B, lq), Cq = shfl_c(Cc, lq), Dq = shfl_c(D, lq);
+        const C k1 = cdiv(A, Bm), k2 = cdiv(Cc, Bq);
+        const C nA = -(k1 * Am), nC = -(k2 * Cq);
+        B = B - k1 * Cm - k2 * Aq;
+        D = D - k1 * Dm - k2 * Dq;
+        A = nA;
+        Cc = nC;
     }
-    const C s = a + c;
-    if (P == 1) return cdiv(d, one + s);
+    if (P == 1) return cdiv(D, A + B + Cc);
     const int lq = lb + ((p + P / 2) & (P - 1));
-    const C sq = shfl_c(s, lq), dq = shfl_c(d, lq);
-    return cdiv(d - s * dq, one - s * sq);
+    const C Aq = shfl_c(A, lq), Bq = shfl_c(B, lq), Cq = shfl_c(Cc, lq), Dq = shfl_c(D, lq);
+    const C apc = A + Cc, aqc = Aq + Cq;
+    return cdiv(D * Bq - apc * Dq, B * Bq - apc * aqc);
 }
 
 // LDS of the reduced systems: first interior values of each chunk (uf, gf,
-// hf), two buffers of normalised interface rows (a, c, d) of which the second
-// takes the place of the first values, and the solutions xi
+// hf) and the interface equations A xi_{p-1} + B xi_p + C xi_{p+1} = D;
+// the solutions overwrite uf
 template <class T>
 struct RedLds {
     static constexpr int kArrays = 7;
-    C2<T> *uf, *gf, *hf, *row, *xi;
-    int n;
-    __device__ __forceinline__ RedLds(C2<T> *base, int n_)
-        : uf(base), gf(base + n_), hf(base + 2 * n_), row(base + 3 * n_), xi(base + 6 * n_), n(n_) {}
+    C2<T> *uf, *gf, *hf, *A, *B, *Cc, *D;
+    __device__ __forceinline__ RedLds(C2<T> *base, int n) {
+        uf = base;
+        gf = uf + n;
+        hf = gf + n;
+        A = hf + n;
+        B = A + n;
+        Cc = B + n;
+        D = Cc + n;
+    }
 };
 
-// interface unknown of chunk p of a line from the chunk's responses and last
-// row (ae, be, ce, de): the cyclic tridiagonal system over the line's P chunk
-// boundaries (chunk q at slot base + q*stride of the LDS arrays) by parallel
-// cyclic reduction until the couplings reach P/2, then 2x2 pairs; the
-// solutions are left in r.xi.  uf, gf and hf are filled and synchronised;
-// every thread of the block calls it.  Normalised rows and two buffers, as in
-// wave_pcr: one barrier and one reciprocal a stage.
+// interface equation of chunk p from its own responses, its last row
+// (ae, be, ce, de) and the first interior values of chunk p+1 at slot nx
 template <class T, int LMAX>
-__device__ __forceinline__ C2<T> interface_solve(const Chunk<T, LMAX> &ck, C2<T> ae, C2<T> be, C2<T> ce, C2<T> de,
-                                                 const RedLds<T> &r, int P, int p, int base, int stride, bool active) {
+__device__ __forceinline__ void interface_row(const Chunk<T, LMAX> &ck, C2<T> ae, C2<T> be, C2<T> ce, C2<T> de,
+                                              const RedLds<T> &r, int nx, C2<T> &A, C2<T> &B, C2<T> &Cv,
+                                              C2<T> &D) {
+    A = ae * ck.gl;
+    B = be + ae * ck.hl + ce * r.gf[nx];
+    Cv = ce * r.hf[nx];
+    D = de - ae * ck.ul - ce * r.uf[nx];
+}
+
+// cyclic tridiagonal system over the P chunk boundaries of one line, held in
+// LDS at slots base + q*stride; every thread of the block must call it.
+// Parallel cyclic reduction until the couplings reach P/2, then 2x2 pairs.
+template <class T>
+__device__ __forceinline__ void reduced_pcr(const RedLds<T> &r, int P, int p, int base, int stride, bool active) {
     using C = C2<T>;
-    const int me = base + p * stride, n = r.n;
-    auto at = [&](int q) { return base + (q & (P - 1)) * stride; };
-    C a{0, 0}, c{0, 0}, d{0, 0}, x{0, 0};
-    C *rd = r.row, *wr = r.uf;
-    if (active) {
-        const int nx = at(p + 1);
-        const C iv = crcp(be + ae * ck.hl + ce * r.gf[nx]);
-        a = (ae * ck.gl) * iv;
-        c = (ce * r.hf[nx]) * iv;
-        d = (de - ae * ck.ul - ce * r.uf[nx]) * iv;
-        rd[me] = a;
-        rd[n + me] = c;
-        rd[2 * n + me] = d;
-    }
-    __syncthreads();
-    const C one{(T)1, (T)0};
+    const int me = base + p * stride;
     for (int st = 1; 2 * st < P; st <<= 1) {
+        C nA{0, 0}, nB{0, 0}, nC{0, 0}, nD{0, 0};
         if (active) {
-            const int im = at(p - st), iq = at(p + st);
-            const C am = rd[im], cm = rd[n + im], dm = rd[2 * n + im];
-            const C aq = rd[iq], cq = rd[n + iq], dq = rd[2 * n + iq];
-            const C iv = crcp(one - a * cm - c * aq);
-            d = (d - a * dm - c * dq) * iv;
-            a = -(a * am) * iv;
-            c = -(c * cq) * iv;
-            wr[me] = a;
-            wr[n + me] = c;
-            wr[2 * n + me] = d;
+            const int im = base + ((p - st) & (P - 1)) * stride, iq = base + ((p + st) & (P - 1)) * stride;
+            const C k1 = cdiv(r.A[me], r.B[im]), k2 = cdiv(r.Cc[me], r.B[iq]);
+            nA = -(k1 * r.A[im]);
+            nC = -(k2 * r.Cc[iq]);
+            nB = r.B[me] - k1 * r.Cc[im] - k2 * r.A[iq];
+            nD = r.D[me] - k1 * r.D[im] - k2 * r.D[iq];
         }
         __syncthreads();
-        C *t = rd;
-        rd = wr;
-        wr = t;
+        if (active) {
+            r.A[me] = nA;
+            r.B[me] = nB;
+            r.Cc[me] = nC;
+            r.D[me] = nD;
+        }
+        __syncthreads();
     }
     if (active) {
-        const C s = a + c;
+        C xi;
         if (P == 1) {
-            x = cdiv(d, one + s);
+            xi = cdiv(r.D[me], r.A[me] + r.B[me] + r.Cc[me]);
         } else {
-            const int q = at(p + P / 2);
-            x = cdiv(d - s * rd[2 * n + q], one - s * (rd[q] + rd[n + q]));
+            const int q = base + ((p + P / 2) & (P - 1)) * stride;
+            const C apc = r.A[me] + r.Cc[me], aqc = r.A[q] + r.Cc[q];
+            xi = cdiv(r.D[me] * r.B[q] - apc * r.D[q], r.B[me] * r.B[q] - apc * aqc);
         }
-        r.xi[me] = x;
+        r.uf[me] = xi;
     }
     __syncthreads();
-    return x;
 }
 
 // (row, column) of flat element e + step of rows of length M, from those of e
@@ -1756,7 +1750,7 @@ __global__ __launch_bounds__(512) void k_xsolve(const C2<T> *__restrict__ src, C
     const int64_t xrow = ((((int64_t)slot * 2 + tcomp) * 3) * g.My + min(y, g.My - 1)) * SL;
     const int64_t xstride = (int64_t)g.My * SL;
     const C *xa = xt + xrow, *xb = xa + xstride, *xc = xb + xstride;
-    const int me = line * P + p;
+    const int me = line * P + p, nx = line * P + ((p + 1) & (P - 1));
     Chunk<T, LMAX> ck;
     ck.uf = ck.gf = ck.hf = ck.ul = ck.gl = ck.hl = C{0, 0};
     if (active) {
@@ -1791,16 +1785,22 @@ __global__ __launch_bounds__(512) void k_xsolve(const C2<T> *__restrict__ src, C
             red.hf[me] = ck.hf;
         }
         __syncthreads();
-        C ae{0, 0}, be{0, 0}, ce{0, 0}, de{0, 0};
+        C A{0, 0}, B{0, 0}, Cv{0, 0}, D{0, 0};
         if (active) {
             const int q = n * P + p;
-            ae = xa[q];
-            be = xb[q];
-            ce = xc[q];
-            de = sdl[q];
+            interface_row(ck, xa[q], xb[q], xc[q], sdl[q], red, nx, A, B, Cv, D);
         }
-        xi = interface_solve(ck, ae, be, ce, de, red, P, p, line * P, 1, active);
-        xprev = red.xi[line * P + ((p - 1) & (P - 1))];
+        __syncthreads();
+        if (active) {
+            red.A[me] = A;
+            red.B[me] = B;
+            red.Cc[me] = Cv;
+            red.D[me] = D;
+        }
+        __syncthreads();
+        reduced_pcr(red, P, p, line * P, 1, active);
+        xi = red.uf[me];
+        xprev = red.uf[line * P + ((p - 1) & (P - 1))];
     }
     if (active) {
         chunk_rebuild(ck, n, xprev, xi, [&](int i, C v) { sdl[i * P + p] = v; });
@@ -1982,7 +1982,7 @@ __global__ __launch_bounds__(512) void k_ysolve(const C2<T> *__restrict__ src, C
         b = C{(T)1 - vb.x, -vb.y};
         c = C{-vc.x, -vc.y};
     };
-    const int me = rb + p * W + cofs;
+    const int me = rb + p * W + cofs, nx = rb + ((p + 1) & (P - 1)) * W + cofs;
     Chunk<T, LMAX> ck;
     if (active) {
         chunk_eliminate<T, LMAX, prefetch_rows<T, LMAX, LEAN>()>(ck, n, [&](int i, C &a, C &b, C &c, C &d) {
@@ -1994,14 +1994,23 @@ __global__ __launch_bounds__(512) void k_ysolve(const C2<T> *__restrict__ src, C
         red.hf[me] = ck.hf;
     }
     __syncthreads();
-    C ae{0, 0}, be{0, 0}, ce{0, 0}, de{0, 0};
+    C A{0, 0}, B{0, 0}, Cv{0, 0}, D{0, 0};
     if (active) {
+        C ae, be, ce;
         tri(s + n, ae, be, ce);
-        de = sd[(n * P + p) * W + cofs];
+        interface_row(ck, ae, be, ce, sd[(n * P + p) * W + cofs], red, nx, A, B, Cv, D);
     }
-    const C xi = interface_solve(ck, ae, be, ce, de, red, P, p, rb + cofs, W, active);
+    __syncthreads();
     if (active) {
-        const C xprev = red.xi[rb + ((p - 1) & (P - 1)) * W + cofs];
+        red.A[me] = A;
+        red.B[me] = B;
+        red.Cc[me] = Cv;
+        red.D[me] = D;
+    }
+    __syncthreads();
+    reduced_pcr(red, P, p, rb + cofs, W, active);
+    if (active) {
+        const C xi = red.uf[me], xprev = red.uf[rb + ((p - 1) & (P - 1)) * W + cofs];
         chunk_rebuild(ck, n, xprev, xi, [&](int i, C v) { sd[(i * P + p) * W + cofs] = v; });
         sd[(n * P + p) * W + cofs] = xi;
     }
@@ -2132,7 +2141,7 @@ __global__ __launch_bounds__(512) void k_ysolve_pair(const C2<T> *__restrict__ s
         b = C{(T)1 - vb.x, -vb.y};
         c = C{-vc.x, -vc.y};
     };
-    const int base = pol * WP + cofs, me = base + p * W;
+    const int base = pol * WP + cofs, me = base + p * W, nx = base + ((p + 1) & (P - 1)) * W;
     Chunk<T, LMAX> ck;
     if (active) {
         chunk_eliminate<T, LMAX, prefetch_rows<T, LMAX, LEAN>()>(ck, n, [&](int i, C &a, C &b, C &c, C &d) {
@@ -2144,14 +2153,23 @@ __global__ __launch_bounds__(512) void k_ysolve_pair(const C2<T> *__restrict__ s
         red.hf[me] = ck.hf;
     }
     __syncthreads();
-    C ae{0, 0}, be{0, 0}, ce{0, 0}, de{0, 0};
+    C A{0, 0}, B{0, 0}, Cv{0, 0}, D{0, 0};
     if (active) {
+        C ae, be, ce;
         tri(s + n, ae, be, ce);
-        de = sdl[(n * P + p) * W + cofs];
+        interface_row(ck, ae, be, ce, sdl[(n * P + p) * W + cofs], red, nx, A, B, Cv, D);
     }
-    const C xi = interface_solve(ck, ae, be, ce, de, red, P, p, base, W, active);
+    __syncthreads();
     if (active) {
-        const C xprev = red.xi[base + ((p - 1) & (P - 1)) * W];
+        red.A[me] = A;
+        red.B[me] = B;
+        red.Cc[me] = Cv;
+        red.D[me] = D;
+    }
+    __syncthreads();
+    reduced_pcr(red, P, p, base, W, active);
+    if (active) {
+        const C xi = red.uf[me], xprev = red.uf[base + ((p - 1) & (P - 1)) * W];
         chunk_rebuild(ck, n, xprev, xi, [&](int i, C v) { sdl[(i * P + p) * W + cofs] = v; });
         sdl[(n * P + p) * W + cofs] = xi;
     }
