@@ -26,6 +26,18 @@ namespace {
 
 const double kPi = 3.1415926535897932;
 
+// hipMalloc whose failure leaves nothing behind: no address, and no error that
+// the next launch check would report
+void device_alloc(void **ptr, size_t bytes) {
+    try {
+        HIPCHK(hipMalloc(ptr, bytes));
+    } catch (...) {
+        *ptr = nullptr;
+        (void)hipGetLastError();
+        throw;
+    }
+}
+
 template <class P>
 struct DevBuf {
     P *ptr = nullptr;
@@ -47,7 +59,7 @@ struct DevBuf {
         release();
         if (!n) return;
         if (source) ptr = static_cast<P *>(source->allocate(n * sizeof(P)));
-        else HIPCHK(hipMalloc((void **)&ptr, n * sizeof(P)));
+        else device_alloc((void **)&ptr, n * sizeof(P));
         count = n;
     }
     // exchanges the allocations of two buffers of the same source
@@ -183,8 +195,9 @@ public:
             own_stream_ = true;
         }
         sz_ = sizes_of(p, o);
-        bind_source(o.allocator, bulk_, bt_, lc_, weights_, q_, iso_t_, iso_n_, partials_, mask_, twx_, twy_, E_, sp_, pp_, cf_,
-                    xt_, fb_[0], fb_[1], fb_[2], fb_[3], flag_, mat_, phase_);
+        bind_source(o.allocator, bulk_, bt_, lc_, weights_, q_, iso_t_, iso_n_, partials_, mask_, twx_, twy_, E_, sp_, pp_,
+                    fb_[0], fb_[1], fb_[2], fb_[3], flag_);
+        solver_.bind(o.allocator);
         g_.Nx = p.Nx;
         g_.Ny = p.Ny;
         g_.Nz = p.Nz;
@@ -302,8 +315,8 @@ public:
     int64_t footprint() const override {
         size_t b = lc_.footprint() + weights_.footprint() + q_.footprint() + iso_t_.footprint() + iso_n_.footprint() +
                    partials_.footprint() + mask_.footprint() + twx_.footprint() + twy_.footprint() +
-                   E_.footprint() + sp_.footprint() + pp_.footprint() + cf_.footprint() + xt_.footprint() +
-                   bulk_.footprint() + bt_.footprint() + flag_.footprint() + mat_.footprint() + phase_.footprint();
+                   E_.footprint() + sp_.footprint() + pp_.footprint() + solver_.footprint() +
+                   bulk_.footprint() + bt_.footprint() + flag_.footprint();
         for (auto &f : fb_) b += f.footprint();
         return (int64_t)b;
     }
@@ -316,6 +329,9 @@ public:
     void download(c64 *E_host) override { staged_d2h(E_host, E_p_, out_bytes(), st_); }
 
     void propagate(Stats *stats) override {
+        if (!solver_ready_)
+            throw BpmError("the context lost its solver buffers to a retune that ran out of device memory: set a "
+                           "tuning again");
         // no_timing: no events at all (the run creates no HIP objects); the
         // stage times stay 0 and the stream is synchronised instead
         const bool timing = !o_.no_timing;
@@ -402,9 +418,39 @@ private:
     std::vector<c64> htwx_, htwy_;
     DevBuf<SlotParams> sp_;
     DevBuf<PropParams> pp_;
-    DevBuf<C2<T>> cf_, xt_;        // stored stencils and x-line rows
-    DevBuf<c64> mat_;              // slab material, both axis orders (walking solvers)
-    DevBuf<C2<T>> phase_;          // phase operators beside it
+    // values of the line solvers' buffers: stored stencils and x-line rows, or
+    // (walking solvers) the slab material in both axis orders and the phase
+    // operators beside it
+    struct SolverCounts {
+        size_t cf = 0, xt = 0, mat = 0, phase = 0;
+    };
+    struct SolverBuffers {
+        DevBuf<C2<T>> cf, xt, phase;
+        DevBuf<c64> mat;
+        void bind(DeviceAllocator *a) { bind_source(a, cf, xt, phase, mat); }
+        SolverCounts counts() const { return {cf.count, xt.count, mat.count, phase.count}; }
+        size_t footprint() const { return cf.footprint() + xt.footprint() + mat.footprint() + phase.footprint(); }
+        // buffers of at least n values wherever o has fewer
+        void alloc_beside(const SolverBuffers &o, const SolverCounts &n) {
+            if (n.cf > o.cf.count) cf.alloc(n.cf);
+            if (n.xt > o.xt.count) xt.alloc(n.xt);
+            if (n.mat > o.mat.count) mat.alloc(n.mat);
+            if (n.phase > o.phase.count) phase.alloc(n.phase);
+        }
+        // takes over what `fresh` holds and gives back what n leaves out
+        void adopt(SolverBuffers &fresh, const SolverCounts &n) {
+            auto one = [](auto &to, auto &from, size_t need) {
+                if (from.ptr) to.swap(from);
+                else if (!need) to.release();
+            };
+            one(cf, fresh.cf, n.cf);
+            one(xt, fresh.xt, n.xt);
+            one(mat, fresh.mat, n.mat);
+            one(phase, fresh.phase, n.phase);
+        }
+    };
+    SolverBuffers solver_;
+    bool solver_ready_ = false;    // solver_ holds the buffers of the shapes in use
     bool walk_ = false;            // the walking solvers march
     WalkShape wx_{}, wy_{};
     DevBuf<C2<T>> fb_[4];
@@ -620,11 +666,11 @@ private:
     C2<T> *march_launches(int nslots, int nprops) {
         const int nsl = p_.Nz - 1, R = sz_.ring, CB = sz_.coef_batch;
         const size_t cfsz = (size_t)sz_.nslots_max * cf_slot_size(g_.Mx, g_.My);
-        const size_t xtsz = xt_.count / R;
+        const size_t xtsz = solver_.xt.count / R;
         // what the boundary reads of slab k: its coefficient tiles, or its phase planes
         auto CF = [&](int k) {
-            return walk_ ? phase_.ptr + (size_t)(k % R) * (size_t)sz_.nslots_max * 3 * sz_.NP
-                         : cf_.ptr + (size_t)(k % R) * cfsz;
+            return walk_ ? solver_.phase.ptr + (size_t)(k % R) * (size_t)sz_.nslots_max * 3 * sz_.NP
+                         : solver_.cf.ptr + (size_t)(k % R) * cfsz;
         };
         const bool overlap = st2_ != nullptr && !walk_ && !tune_.coef_serial;
         const WalkRing<T> ring = walk_ring();
@@ -644,8 +690,8 @@ private:
                     launch_slab_material<T>(lc_p_, mask_p_, w_p_, g_, sp_.ptr, nslots, k0, n, ring, R, s);
                     return;
                 }
-                launch_slab_coefs<T>(lc_p_, mask_p_, w_p_, g_, sp_.ptr, nslots, k0, n, cf_.ptr, (int64_t)cfsz,
-                                     xt_.ptr, (int64_t)xtsz, R, lpx_, s);
+                launch_slab_coefs<T>(lc_p_, mask_p_, w_p_, g_, sp_.ptr, nslots, k0, n, solver_.cf.ptr, (int64_t)cfsz,
+                                     solver_.xt.ptr, (int64_t)xtsz, R, lpx_, s);
             });
         };
         auto coef = [&](int k) {
@@ -714,7 +760,7 @@ private:
     // both half-steps of slab k on its stored stencils cf: cur -> cur (y slow)
     void planes_slab(int k, int nprops, C2<T> *cur, C2<T> *other, C2<T> *A, C2<T> *B, const C2<T> *cf) {
         const int nw = p_.n_woodbury;
-        const C2<T> *xt = xt_.ptr ? xt_.ptr + (size_t)(k % sz_.ring) * (xt_.count / sz_.ring) : nullptr;
+        const C2<T> *xt = solver_.xt.ptr ? solver_.xt.ptr + (size_t)(k % sz_.ring) * (solver_.xt.count / sz_.ring) : nullptr;
         // XCD work order (measured): a lone polarisation pair shares L2 best
         // across the two components; batches whose field planes total up to
         // about 32 MiB do best with the pairs innermost (the wavevectors of a
@@ -769,9 +815,9 @@ private:
     WalkRing<T> walk_ring() const {
         WalkRing<T> r{};
         if (!walk_) return r;
-        r.mat = mat_.ptr;
+        r.mat = solver_.mat.ptr;
         r.mat_stride = mat_slab();
-        r.phase = phase_.ptr;
+        r.phase = solver_.phase.ptr;
         r.phase_stride = (size_t)sz_.nslots_max * 3 * sz_.NP;
         return r;
     }
@@ -821,9 +867,7 @@ private:
     }
 
     // Validates the shapes asked for, then switches to them (the runner keeps
-    // its state when they are refused).  The captured graphs hold the buffer
-    // pointers of the old shapes, so they are destroyed before any buffer
-    // changes.
+    // its shapes when they are refused or their buffers do not fit).
     //
     // FP64 marches at the built-in shapes take the walking solvers wherever
     // they have a shape (both axes periodic, march lines of 16 to 1024
@@ -842,10 +886,10 @@ private:
             wy = walk_shape(g_.My, g_.Mx, sz_.nprops_max);
         }
         if (wx.W > 0 && wy.W > 0) {
-            drop_graphs();
-            cf_.release();
-            xt_.release();
-            alloc_walk();
+            SolverCounts n;
+            n.mat = (size_t)sz_.ring * mat_slab();
+            n.phase = (size_t)sz_.ring * sz_.nslots_max * 3 * sz_.NP;
+            hold_buffers(n);
             walk_ = true;
             wx_ = wx;
             wy_ = wy;
@@ -861,39 +905,55 @@ private:
         if (g_.py && ((t.y_pair ? 2 : 1) * ly.P * t.y_cols > 512 ||
                       ysolve_lds_bytes<T>(ly, t.y_cols, t.y_pair) > max_block_lds()))
             throw std::runtime_error("y line solver tuning exceeds the block limits");
-        drop_graphs();
-        mat_.release();
-        phase_.release();
-        try {
-            if (!cf_.ptr) cf_.alloc((size_t)sz_.ring * sz_.nslots_max * cf_slot_size(g_.Mx, g_.My));
-            if (g_.px) {
-                // a larger x-line row buffer is allocated beside the old one
-                const size_t need = (size_t)sz_.ring * sz_.nslots_max * 2 * 3 * g_.My * lx.lmax * lx.P;
-                if (need > xt_.count) {
-                    DevBuf<C2<T>> grown;
-                    grown.source = xt_.source;
-                    grown.alloc(need);
-                    xt_.swap(grown);  // the old rows are released with `grown`
-                }
-            }
-        } catch (...) {
-            if (walk_) {
-                cf_.release();
-                xt_.release();
-                alloc_walk();
-            }
-            throw;
-        }
+        SolverCounts n;
+        n.cf = (size_t)sz_.ring * sz_.nslots_max * cf_slot_size(g_.Mx, g_.My);
+        if (g_.px) n.xt = (size_t)sz_.ring * sz_.nslots_max * 2 * 3 * g_.My * lx.lmax * lx.P;
+        hold_buffers(n);
         walk_ = false;
         tune_ = t;
         lpx_ = lx;
         lpy_ = ly;
     }
 
-    void alloc_walk() {
-        if (mat_.ptr) return;
-        mat_.alloc((size_t)sz_.ring * mat_slab());
-        phase_.alloc((size_t)sz_.ring * sz_.nslots_max * 3 * sz_.NP);
+    // Brings the line solvers' buffers to n values, all of them or none: the
+    // new ones are taken beside the old (a buffer that is large enough stays).
+    // Where the device cannot hold both, the old ones are given back first,
+    // and taken again if the new ones still do not fit.  If even that fails,
+    // another user of the device having taken the memory, the runner is left
+    // without and refuses to march until a retune succeeds.
+    void hold_buffers(const SolverCounts &n) {
+        auto take = [&] {
+            SolverBuffers fresh;
+            fresh.bind(o_.allocator);
+            fresh.alloc_beside(solver_, n);
+            drop_graphs();  // (they hold the old pointers)
+            solver_.adopt(fresh, n);
+            solver_ready_ = true;
+        };
+        try {
+            take();
+            return;
+        } catch (const std::exception &) {
+            if (!solver_ready_) throw;
+        }
+        const SolverCounts had = solver_.counts();
+        drop_graphs();
+        solver_ready_ = false;
+        SolverBuffers none;
+        solver_.adopt(none, SolverCounts());
+        try {
+            take();
+        } catch (...) {
+            try {
+                SolverBuffers again;
+                again.bind(o_.allocator);
+                again.alloc_beside(solver_, had);
+                solver_.adopt(again, had);
+                solver_ready_ = true;
+            } catch (const std::exception &) {
+            }
+            throw;
+        }
     }
 
     void retune(const Tuning &t) override {
