@@ -25,7 +25,7 @@
 // 1024^2 120-125 us (130-156 / 225-238).  Per slab, whole march: 64^2 54 us
 // (68), 161^2 74 us (96), 128^2 x 7 pairs 109 us (120), x 147 pairs 1.27 ms
 // (1.46), 256^2 x 147 pairs 5.5 ms (6.2).  A whole 512^2 x 100 propagation
-// 25.1 -> 17.5 ms, 1024^2 x 200 267.5 -> 171.5 ms.
+// 25.1 -> 17.3 ms, 1024^2 x 200 267.5 -> 172.7 ms.
 //
 // Lanes of a wave lie across the lines (consecutive in memory) and chunks of
 // them: the state is kept with the line axis slow, [l][t] for lines along l.
@@ -58,9 +58,11 @@ namespace nmk {
 
 namespace {
 
-// 1/v to the last bit or two: the hardware estimate and two Newton steps (an
-// IEEE division is twice as long a chain, and the eliminations are chains of
-// them); the fix-up gives the special values of the division
+// 1/v: the hardware estimate and two Newton steps (an IEEE division is twice
+// as long a chain, and the eliminations are chains of them: 64^2 x 20 1.106 ms
+// against 1.125, 1024^2 x 200 172.7 against 173.9); the fix-up gives the special
+// values of the division.  Errors of nine marches (64^2 to 300 x 210, droplets,
+// beams, oblique) against long double arithmetic: equal to four digits.
 __device__ __forceinline__ double rcp_newton(double v) {
     double r = __builtin_amdgcn_rcp(v);
     r = fma(r, fma(-v, r, 1.0), r);
@@ -515,9 +517,12 @@ __global__ __launch_bounds__(512) void k_walk(const c64 *__restrict__ src, c64 *
         walk_lines<STEPS, W, NEU, 1>(tid, lp, mat, src + pb, axis, tb, Ml, Mt, (int)NP, rows, p, cc, is_short, st, ck);
     __syncthreads();
 
-    // the interface unknowns of the line's chunks: cyclic tridiagonal, rows normalised to x_p + a x_{p-1} + c x_{p+1}
-    // = d, by cyclic reduction with two LDS buffers of three arrays
-    static_assert(3 * 2 * W * R::P <= R::buffer, "reduced systems");
+    // the interface unknowns of the line's chunks: cyclic tridiagonal, A x_{p-1} + B x_p + C x_{p+1} = D, by cyclic
+    // reduction with two LDS buffers of four arrays.  Each thread inverts its own B once a stage, for its neighbours.
+    // The right-hand side is corrected, never rescaled: rows normalised to B = 1 take six values a stage (1024^2 x 200
+    // 171.5 ms against 172.7, 512^2 x 100 17.2 against 17.3), but there the rounding of every stage reaches the unknowns
+    // in full (error of the former 2.5e-15 against 5.7e-16, as the solvers on stored stencils).
+    static_assert(4 * 2 * W * R::P <= R::buffer, "reduced systems");
     C *buf0 = rows0, *buf1 = rows1;
     buf0[tid] = ck.uf;
     buf0[NT + tid] = ck.gf;
@@ -533,43 +538,44 @@ __global__ __launch_bounds__(512) void k_walk(const c64 *__restrict__ src, c64 *
     __syncthreads();
     const int lb = comp * TW + cc;
     auto at = [&](int q) { return lb + ((q & (P - 1)) << lw); };
-    C a, c, d;
+    C a, b, c, d;
     {
         const int nx = at(p + 1);
         const C ufn = buf0[nx], gfn = buf0[NT + nx], hfn = buf0[2 * NT + nx];
-        const C iv = wrcp(ck.be + ck.ae * ck.hl + ck.ce * gfn);
-        a = (ck.ae * ck.gl) * iv;
-        c = (ck.ce * hfn) * iv;
-        d = (ck.de - ck.ae * ck.ul - ck.ce * ufn) * iv;
+        a = ck.ae * ck.gl;
+        b = ck.be + ck.ae * ck.hl + ck.ce * gfn;
+        c = ck.ce * hfn;
+        d = ck.de - ck.ae * ck.ul - ck.ce * ufn;
     }
-    buf1[tid] = a;
-    buf1[NT + tid] = c;
-    buf1[2 * NT + tid] = d;
-    __syncthreads();
+    // to the other threads of the line: 1/B for a stage of the reduction, B for the last pairs
+    auto publish = [&](C *x, C bv) {
+        x[tid] = a;
+        x[NT + tid] = bv;
+        x[2 * NT + tid] = c;
+        x[3 * NT + tid] = d;
+        __syncthreads();
+    };
+    publish(buf1, wrcp(b));
     C *rd = buf1, *wr = buf0;
     for (int stp = 1; 2 * stp < P; stp <<= 1) {
         const int im = at(p - stp), iq = at(p + stp);
-        const C am = rd[im], cm = rd[NT + im], dm = rd[2 * NT + im];
-        const C aq = rd[iq], cq = rd[NT + iq], dq = rd[2 * NT + iq];
-        const C iv = wrcp(C{1, 0} - a * cm - c * aq);
-        d = (d - a * dm - c * dq) * iv;
-        a = -(a * am) * iv;
-        c = -(c * cq) * iv;
-        wr[tid] = a;
-        wr[NT + tid] = c;
-        wr[2 * NT + tid] = d;
-        __syncthreads();
+        const C k1 = a * rd[NT + im], k2 = c * rd[NT + iq];
+        const C am = rd[im], cm = rd[2 * NT + im], dm = rd[3 * NT + im];
+        const C aq = rd[iq], cq = rd[2 * NT + iq], dq = rd[3 * NT + iq];
+        a = -(k1 * am);
+        c = -(k2 * cq);
+        b = b - k1 * cm - k2 * aq;
+        d = d - k1 * dm - k2 * dq;
+        publish(wr, 4 * stp < P ? wrcp(b) : b);
         C *x = rd;
         rd = wr;
         wr = x;
     }
     C xi;
-    if (P == 1) {
-        xi = d * wrcp(C{1, 0} + a + c);
-    } else {
+    {
         const int q = at(p + P / 2);
-        const C bq = rd[q] + rd[NT + q], dq = rd[2 * NT + q], b0 = a + c;
-        xi = (d - b0 * dq) * wrcp(C{1, 0} - b0 * bq);
+        const C bq = rd[NT + q], dq = rd[3 * NT + q], b0 = a + c, b1 = rd[q] + rd[2 * NT + q];
+        xi = (d * bq - b0 * dq) * wrcp(b * bq - b0 * b1);
     }
     wr[tid] = xi;
     __syncthreads();
@@ -661,8 +667,8 @@ void launch_walk(int axis, int neumann, const c64 *src, c64 *dst, const c64 *acc
                  int per_slot, const WalkShape &sh, hipStream_t st) {
     const LinePlan &lp = sh.lp;
     const int Ml = axis == 0 ? g.Mx : g.My, Mt = axis == 0 ? g.My : g.Mx;
-    // a wave holds chunks of one component; rows and result of a block fit its LDS buffers
-    if (!g.px || !g.py || lp.M != Ml || 2 * lp.P * sh.W > 512 ||
+    // a wave holds chunks of one component; rows and result of a block fit its LDS buffers; the reduction takes a stage
+    if (!g.px || !g.py || lp.M != Ml || lp.P < 4 || 2 * lp.P * sh.W > 512 ||
         lp.P * sh.W % 64 || per_slot < 1 || nprops % per_slot)
         throw std::runtime_error("line walk: bad launch shape");
     const int64_t items = (int64_t)((Mt + sh.W - 1) / sh.W) * nprops;
