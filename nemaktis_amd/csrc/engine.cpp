@@ -183,6 +183,35 @@ WalkShape walk_shape(int M, int Mt, int nprops) {
     return sh;
 }
 
+// Whether a march of nprops propagations, nq directions a wavelength, is
+// faster with the walking solvers than on stored stencils (850 meshes and
+// batches of 9 to 1024 points an axis timed both ways, us a slab stored ->
+// walking).  The walk generates the stencils for every propagation, reads two
+// columns beside the lines of a block and two rows beside each chunk, and has
+// few lines a block where they are long; the stored ones are shared by the
+// directions of a wavelength, and their y lines are dear where x lines are
+// short, cheap where they are long.
+//   At most one round of blocks on 256 CUs: the walk (64^2 68 -> 54, 191 x 25
+// at 7 directions 75.6 -> 75.7, the least), but on narrow strips along x
+// (505 x 17 73 -> 75, 1000 x 48 116 -> 117; 350 x 24 68 -> 65).
+//   More rounds, one direction: the walk from 64-point y lines (401 x 65 at 7
+// wavelengths 178 -> 149, 1001 x 301 at 3 1079 -> 743; 1001 x 41 at 3 145 ->
+// 159, 601 x 21 at 7 121 -> 139).
+//   Several directions share: from 128-point y lines (600 x 130 at 7
+// directions 505 -> 479, 1000 x 200 1085 -> 1075; 600 x 64 225 -> 256, 1000 x 12
+// at 37 271 -> 583), and beyond a ring of them only where blocks hold many
+// lines along x and not too many rounds along y (200^2 at 37 981 -> 940, 300 x
+// 600 at 19 2540 -> 2320; 1000 x 300 at 37 9020 -> 10930, 256 x 1000 8210 -> 8520,
+// 64 x 1000 1870 -> 2060, 340 x 600 at 61 12380 -> 13020).
+bool walk_pays(int Mx, int My, int nq, int nprops, const WalkShape &wx, const WalkShape &wy) {
+    if (wx.W == 0 || wy.W == 0 || Mx > 16 * My) return false;
+    auto blocks = [&](const WalkShape &w, int Mt) { return (int64_t)((Mt + w.W - 1) / w.W) * nprops; };
+    if (blocks(wx, My) <= 256 && blocks(wy, Mx) <= 256) return true;
+    if (nq == 1) return My >= 64;
+    if (nq <= 7) return My >= 128;
+    return My >= 128 && My <= (nq <= 37 ? 640 : 400) && Mx >= 96 && Mx <= 384;
+}
+
 template <class T>
 class RunnerT final : public Runner {
 public:
@@ -869,11 +898,11 @@ private:
     // Validates the shapes asked for, then switches to them (the runner keeps
     // its shapes when they are refused or their buffers do not fit).
     //
-    // FP64 marches at the built-in shapes take the walking solvers wherever
-    // they have a shape (both axes periodic, march lines of 16 to 1024
-    // points): 25.1 -> 17.5 ms for 512^2 x 100 at one propagation pair, 267.5
-    // -> 171.5 ms for 1024^2 x 200, a slab of 96 x 80 at 70 pairs 371 -> 337
-    // us, of 256^2 at 147 pairs 6.2 -> 5.5 ms.  Explicit shapes are shapes of the
+    // FP64 marches at the built-in shapes take the walking solvers where they
+    // have a shape (both axes periodic, march lines of up to 1024 points) and
+    // pay (walk_pays): 25.1 -> 17.3 ms for 512^2 x 100 at one propagation pair,
+    // 267.5 -> 172.7 ms for 1024^2 x 200, a slab of 256^2 at 147 pairs 6.2 ->
+    // 5.5 ms.  Explicit shapes are shapes of the
     // solvers on stored stencils.  FP32 stays there too: its stencils are half
     // the bytes and shared by the propagations of a wavelength, where the walk
     // generates them for each (256^2 at 147 pairs 771-789 us a launch against
@@ -885,7 +914,7 @@ private:
             wx = walk_shape(g_.Mx, g_.My, sz_.nprops_max);
             wy = walk_shape(g_.My, g_.Mx, sz_.nprops_max);
         }
-        if (wx.W > 0 && wy.W > 0) {
+        if (walk_pays(g_.Mx, g_.My, sz_.nq, sz_.nprops_max, wx, wy)) {
             SolverCounts n;
             n.mat = (size_t)sz_.ring * mat_slab();
             n.phase = (size_t)sz_.ring * sz_.nslots_max * 3 * sz_.NP;

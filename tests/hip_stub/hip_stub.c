@@ -10,11 +10,33 @@ typedef struct { unsigned x, y, z; } dim;
 
 static int last, skip, fail, launches;
 static size_t live;
+static struct { const void *f; char name[256]; } kernels[4096];
+static int nkernels, seen[4096];
 
 /* of the following hipMalloc calls, the first s succeed and the next n fail */
 void stub_fail(int s, int n) { skip = s, fail = n; }
 size_t stub_live(void) { return live; }
 int stub_launches(void) { return launches; }
+/* kernels of the library: the mangled name of kernel i, and whether it was launched since this was last asked */
+int stub_kernels(void) { return nkernels; }
+const char *stub_name(int i) { return kernels[i].name; }
+int stub_seen(int i) {
+    const int v = seen[i];
+    seen[i] = 0;
+    return v;
+}
+void **__hipRegisterFatBinary(const void *b) { return (void)b, (void **)kernels; }
+void __hipUnregisterFatBinary(void **b) { (void)b; }
+void __hipRegisterFunction(void **b, const void *f, char *d, const char *name, unsigned n, void *t, void *bl, void *bd,
+                           void *gd, int *w) {
+    (void)b, (void)d, (void)n, (void)t, (void)bl, (void)bd, (void)gd, (void)w;
+    if (nkernels == 4096) abort();
+    kernels[nkernels].f = f;
+    strncpy(kernels[nkernels++].name, name, 255);
+}
+void __hipRegisterVar(void **b, void *v, char *h, char *d, int e, size_t n, int c, int g) {
+    (void)b, (void)v, (void)h, (void)d, (void)e, (void)n, (void)c, (void)g;
+}
 
 int hipMalloc(void **p, size_t n) {
     *p = NULL;
@@ -40,7 +62,9 @@ int hipFree(void *p) {
     return OK;
 }
 int hipLaunchKernel(const void *f, dim g, dim b, void **args, size_t lds, void *st) {
-    (void)f, (void)g, (void)b, (void)args, (void)lds, (void)st;
+    (void)g, (void)b, (void)args, (void)lds, (void)st;
+    for (int i = 0; i < nkernels; i++)
+        if (kernels[i].f == f) seen[i] = 1;
     launches++;
     return OK;
 }

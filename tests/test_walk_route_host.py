@@ -1,0 +1,97 @@
+"""Which line solvers an FP64 march at the built-in shapes takes: the walking
+ones where they were measured to be the faster (walk_pays in engine.cpp), the
+ones on stored stencils elsewhere.  The library runs on the stand-in for the
+HIP runtime (hip_stub/hip_stub.c), which notes the kernels launched."""
+import json
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+# mesh, directions a wavelength, wavelengths, precision; True: walks.  Times a slab in us, stored / walking
+ROUTES = [
+    ((65, 65), 1, 1, 64, True),        # 68 / 54
+    ((512, 512), 1, 1, 64, True),      # 252 / 173
+    ((512, 512), 1, 1, 32, False),     # FP32 keeps the stored stencils
+    ((128, 128), 7, 1, 64, True),      # one round of blocks: 120 / 109
+    ((192, 26), 7, 1, 64, True),       # 75.6 / 75.7
+    ((506, 18), 1, 1, 64, False),      # 73.1 / 74.8
+    ((1000, 17), 1, 1, 64, False),     # 94.5 / 96.1
+    ((1001, 49), 1, 1, 64, False),     # 115.8 / 117
+    ((339, 19), 1, 1, 64, False),      # 68 / 64, left out with the strips
+    ((351, 25), 1, 1, 64, True),       # 68.1 / 64.7
+    ((18, 506), 1, 1, 64, True),
+    ((401, 66), 1, 7, 64, True),       # 178 / 149
+    ((1001, 41), 1, 3, 64, False),     # 145 / 159
+    ((601, 21), 1, 7, 64, False),      # 121 / 139
+    ((13, 1001), 1, 7, 64, True),      # 232 / 163
+    ((1001, 13), 1, 7, 64, False),     # 124 / 163
+    ((601, 131), 7, 1, 64, True),      # 505 / 479
+    ((1001, 201), 7, 1, 64, True),     # 1085 / 1075
+    ((601, 65), 7, 1, 64, False),      # 225 / 256
+    ((301, 41), 7, 1, 64, False),      # 113 / 125
+    ((1000, 12), 37, 1, 64, False),    # 271 / 583
+    ((201, 201), 37, 1, 64, True),     # 981 / 940
+    ((301, 601), 19, 1, 64, True),     # 2540 / 2320
+    ((341, 601), 61, 1, 64, False),    # 12380 / 13020
+    ((385, 301), 61, 1, 64, True),     # 5500 / 5170
+    ((1001, 301), 37, 1, 64, False),   # 9020 / 10930
+    ((257, 1001), 37, 1, 64, False),   # 8210 / 8520
+    ((65, 1001), 37, 1, 64, False),    # 1870 / 2060
+    ((1026, 65), 1, 1, 64, False),     # no shape above 1024 points
+    ((8, 65), 1, 1, 64, False),        # nor below 8
+    ((9, 65), 1, 1, 64, True),
+    ((3, 65), 1, 1, 64, False),        # an axis that is not periodic
+]
+
+DRIVER = """
+import ctypes, json, sys
+stub = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+stub.stub_name.restype = ctypes.c_char_p
+sys.path.insert(0, sys.argv[2])
+import numpy as np
+from nemaktis_amd import bpm_backend, fields
+
+for (nx, ny), nq, nwl, precision, _ in json.loads(sys.argv[3]):
+    dims = (nx, ny, 2)
+    s = fields.make_settings(dims, (0.1, 0.1, 0.1), [0.5 + 0.01 * k for k in range(nwl)],
+                             wavevectors=[(0.01 * k, 0.0) for k in range(nq)])
+    lc = np.zeros((2 * nx * ny, 3))
+    with bpm_backend.Context(json.dumps(s), lc, int(np.prod(fields.output_shape(s))), precision=precision,
+                             wl_batch=0) as c:
+        c.propagate()
+    names = [stub.stub_name(i).decode() for i in range(stub.stub_kernels()) if stub.stub_seen(i)]
+    print("route", json.dumps(names))
+"""
+
+
+def launched(so, jobs):
+    """The mangled names of the kernels that each job launches."""
+    r = subprocess.run([sys.executable, "-c", DRIVER, so, ROOT, json.dumps(jobs)], stdout=subprocess.PIPE,
+                       stderr=subprocess.STDOUT, text=True, timeout=600)
+    assert r.returncode == 0, r.stdout[-3000:]
+    return [json.loads(line[6:]) for line in r.stdout.splitlines() if line.startswith("route ")]
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    if not shutil.which("gcc"):
+        pytest.skip("gcc is not available")
+    so = str(tmp_path_factory.mktemp("stub") / "libhip_stub.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-o", so, os.path.join(ROOT, "tests", "hip_stub", "hip_stub.c")],
+                   check=True)
+    return so
+
+
+def test_routes(stub):
+    got = []
+    for job, names in zip(ROUTES, launched(stub, ROUTES)):
+        walks = any("k_walk" in n for n in names)
+        stored = any("k_xsolve" in n or "k_ysolve" in n for n in names)
+        assert walks != stored, (job, names)
+        got.append(job[:4] + (walks,))
+    assert got == ROUTES
