@@ -715,9 +715,8 @@ private:
         // coefficients of slabs k0 .. k0+n-1 in one launch on stream s
         auto coefs = [&](int k0, int n, hipStream_t s) {
             timed(KF_COEFS, [&] {
-                if (walk_) {
-                    launch_slab_material<T>(lc_p_, mask_p_, w_p_, g_, sp_.ptr, nslots, k0, n, ring, R, s);
-                    return;
+                if constexpr (sizeof(T) == 8) {
+                    if (walk_) return launch_slab_material<T>(lc_p_, mask_p_, w_p_, g_, sp_.ptr, nslots, k0, n, ring, R, s);
                 }
                 launch_slab_coefs<T>(lc_p_, mask_p_, w_p_, g_, sp_.ptr, nslots, k0, n, solver_.cf.ptr, (int64_t)cfsz,
                                      solver_.xt.ptr, (int64_t)xtsz, R, lpx_, s);

@@ -14,6 +14,7 @@
 #include <cmath>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "kernels.h"
@@ -723,6 +724,17 @@ static inline unsigned tiles_for(int nx, int ny) {
     return (unsigned)(((nx + kWalkTile - 1) / kWalkTile) * ((ny + kWalkTile - 1) / kWalkTile));
 }
 
+// launches f(std::true_type) for a state with x slow, else f(std::false_type);
+// only FP64 marches keep it so
+template <class T, class F>
+static void by_order(bool x_slow, F &&f) {
+    if constexpr (sizeof(T) == 8) {
+        if (x_slow) return f(std::true_type{});
+    }
+    if (x_slow) throw std::runtime_error("a state with x slow is FP64");
+    f(std::false_type{});
+}
+
 // ---------------------------------------------------------------------------
 // input beam (PhysicsLib/BeamProfile.cpp:17-39) + input Fresnel
 // (BeamPropagationLib/FresnelOperator.cpp:16-38), written to the march grid
@@ -813,12 +825,11 @@ template <class T>
 void launch_init_fields(const double *lc, const uint8_t *mask, const Geo &g, const SlotParams *sp,
                         const PropParams *pp, int nprops, int gaussian, double waist, double dx, double dy,
                         C2<T> *F, bool x_slow, hipStream_t st) {
-    if (x_slow)
-        hipLaunchKernelGGL((k_init_fields<T, true>), dim3(tiles_for(g.Mx, g.My), nprops), dim3(256), 0, st, lc, mask,
-                           g, sp, pp, gaussian, waist, dx, dy, F);
-    else
-        hipLaunchKernelGGL((k_init_fields<T, false>), dim3(blocks_for(g.NP, 256), nprops), dim3(256), 0, st, lc, mask,
-                           g, sp, pp, gaussian, waist, dx, dy, F);
+    by_order<T>(x_slow, [&](auto xs) {
+        const unsigned blocks = xs ? tiles_for(g.Mx, g.My) : blocks_for(g.NP, 256);
+        hipLaunchKernelGGL((k_init_fields<T, decltype(xs)::value>), dim3(blocks, nprops), dim3(256), 0, st, lc, mask, g,
+                           sp, pp, gaussian, waist, dx, dy, F);
+    });
     NMK_LAUNCH_CHECK();
 }
 
@@ -844,10 +855,10 @@ void launch_pack_fields(const c64 *E, const Geo &g, const PropParams *pp, int np
                         bool x_slow, hipStream_t st) {
     (void)pp;
     (void)nq;
-    if (x_slow)
-        hipLaunchKernelGGL((k_pack_fields<T, true>), dim3(tiles_for(g.Mx, g.My), nprops), dim3(256), 0, st, E, g, F);
-    else
-        hipLaunchKernelGGL((k_pack_fields<T, false>), dim3(blocks_for(g.NP, 256), nprops), dim3(256), 0, st, E, g, F);
+    by_order<T>(x_slow, [&](auto xs) {
+        const unsigned blocks = xs ? tiles_for(g.Mx, g.My) : blocks_for(g.NP, 256);
+        hipLaunchKernelGGL((k_pack_fields<T, decltype(xs)::value>), dim3(blocks, nprops), dim3(256), 0, st, E, g, F);
+    });
     NMK_LAUNCH_CHECK();
 }
 
@@ -1084,15 +1095,16 @@ void launch_boundary(const C2<T> *in, C2<T> *out, const C2<T> *cf_prev, const C2
         std::swap(e.Mx, e.My);
         std::swap(e.px, e.py);
     }
-    if (unshifted) {
-        dim3 grid((unsigned)blocks_for(g.NP, 256), nprops / 2);
-        if (x_slow) hipLaunchKernelGGL((k_boundary_point<T, true>), grid, dim3(256), 0, st, in, out, cf_prev, cf_next, e, pp);
-        else hipLaunchKernelGGL((k_boundary_point<T, false>), grid, dim3(256), 0, st, in, out, cf_prev, cf_next, e, pp);
-    } else {
-        dim3 grid((e.Mx + kBTW - 1) / kBTW, (e.My + kBTH - 1) / kBTH, nprops / 2);
-        if (x_slow) hipLaunchKernelGGL((k_boundary<T, true>), grid, dim3(256), 0, st, in, out, cf_prev, cf_next, e, pp, nshift);
-        else hipLaunchKernelGGL((k_boundary<T, false>), grid, dim3(256), 0, st, in, out, cf_prev, cf_next, e, pp, nshift);
-    }
+    by_order<T>(x_slow, [&](auto xs) {
+        constexpr bool XS = decltype(xs)::value;
+        if (unshifted) {
+            dim3 grid((unsigned)blocks_for(g.NP, 256), nprops / 2);
+            hipLaunchKernelGGL((k_boundary_point<T, XS>), grid, dim3(256), 0, st, in, out, cf_prev, cf_next, e, pp);
+        } else {
+            dim3 grid((e.Mx + kBTW - 1) / kBTW, (e.My + kBTH - 1) / kBTH, nprops / 2);
+            hipLaunchKernelGGL((k_boundary<T, XS>), grid, dim3(256), 0, st, in, out, cf_prev, cf_next, e, pp, nshift);
+        }
+    });
     NMK_LAUNCH_CHECK();
 }
 
@@ -2428,12 +2440,11 @@ template <class T>
 void launch_output(const C2<T> *F, const double *lc, const uint8_t *mask, const Geo &g, const SlotParams *sp,
                    const PropParams *pp, int nprops, int nq, c64 *E, bool x_slow, hipStream_t st) {
     (void)nq;
-    if (x_slow)
-        hipLaunchKernelGGL((k_output<T, true>), dim3(tiles_for(g.Nx, g.Ny), nprops), dim3(256), 0, st, F, lc, mask, g,
+    by_order<T>(x_slow, [&](auto xs) {
+        const unsigned blocks = xs ? tiles_for(g.Nx, g.Ny) : blocks_for(g.Nfull, 256);
+        hipLaunchKernelGGL((k_output<T, decltype(xs)::value>), dim3(blocks, nprops), dim3(256), 0, st, F, lc, mask, g,
                            sp, pp, E);
-    else
-        hipLaunchKernelGGL((k_output<T, false>), dim3(blocks_for(g.Nfull, 256), nprops), dim3(256), 0, st, F, lc, mask,
-                           g, sp, pp, E);
+    });
     NMK_LAUNCH_CHECK();
 }
 
@@ -2522,12 +2533,11 @@ __global__ __launch_bounds__(256) void k_bulk_plane(const C2<T> *__restrict__ F,
 template <class T>
 void launch_bulk_plane(const C2<T> *F, const Geo &g, const SlotParams *sp, const PropParams *pp, int nprops,
                        int plane, int nq, c64 *bulk, bool x_slow, hipStream_t st) {
-    if (x_slow)
-        hipLaunchKernelGGL((k_bulk_plane<T, true>), dim3(tiles_for(g.Nx, g.Ny), nprops), dim3(256), 0, st, F, g, sp, pp,
+    by_order<T>(x_slow, [&](auto xs) {
+        const unsigned blocks = xs ? tiles_for(g.Nx, g.Ny) : blocks_for(g.Nfull, 256);
+        hipLaunchKernelGGL((k_bulk_plane<T, decltype(xs)::value>), dim3(blocks, nprops), dim3(256), 0, st, F, g, sp, pp,
                            plane, nq, bulk);
-    else
-        hipLaunchKernelGGL((k_bulk_plane<T, false>), dim3(blocks_for(g.Nfull, 256), nprops), dim3(256), 0, st, F, g, sp,
-                           pp, plane, nq, bulk);
+    });
     NMK_LAUNCH_CHECK();
 }
 
@@ -2839,8 +2849,6 @@ void launch_filter(c64 *E, const Geo &g, const SlotParams *sp, int nslots, const
     template void launch_init_fields<T>(const double *, const uint8_t *, const Geo &, const SlotParams *,             \
                                         const PropParams *, int, int, double, double, double, C2<T> *, bool,        \
                                         hipStream_t);                                                                \
-    template void launch_slab_material<T>(const double *, const uint8_t *, const double *, const Geo &,            \
-                                          const SlotParams *, int, int, int, const WalkRing<T> &, int, hipStream_t);  \
     template void launch_pack_fields<T>(const c64 *, const Geo &, const PropParams *, int, int, C2<T> *, bool,      \
                                         hipStream_t);                                                                \
     template void launch_boundary<T>(const C2<T> *, C2<T> *, const C2<T> *, const C2<T> *, const Geo &,             \
@@ -2860,5 +2868,8 @@ void launch_filter(c64 *E, const Geo &g, const SlotParams *sp, int nslots, const
                                    const PropParams *, int, int, c64 *, bool, hipStream_t);
 NMK_INST(float)
 NMK_INST(double)
+template void launch_slab_material<double>(const double *, const uint8_t *, const double *, const Geo &,
+                                           const SlotParams *, int, int, int, const WalkRing<double> &, int,
+                                           hipStream_t);
 
 }  // namespace nmk

@@ -627,13 +627,13 @@ __global__ __launch_bounds__(512) void k_walk(const c64 *__restrict__ src, c64 *
             if (i + 1 < STEPS || !is_short) row[(s0 + i) + ((s0 + i) >> 3)] = ck.yu[i];
     }
     __syncthreads();
-    const int ws = min(64, NT), lane = tid & (ws - 1), wave = tid / ws, nwave = NT / ws;  // NT is a power of two
+    const int lane = tid & 63, wave = tid >> 6, nwave = NT >> 6;
     for (int q = wave; q < 2 * W; q += nwave) {
         const int qc = q >> lw, to = tb + (q & (W - 1));
         if (to >= Mt) continue;
         C *o = acc + pb + (size_t)(qc == (axis == 0 ? 0 : 1) ? 0 : 1) * NP + (size_t)to * Ml;
         const C *row = (qc == 0 ? rows0 : rows1) + (q & (W - 1)) * ld;
-        for (int l = lane; l < Ml; l += ws) o[l] = row[l + (l >> 3)];
+        for (int l = lane; l < Ml; l += 64) o[l] = row[l + (l >> 3)];
     }
 }
 
@@ -643,11 +643,15 @@ static void walk_dispatch(const WalkShape &sh, dim3 grid, const c64 *src, c64 *d
                           const PropParams *pp, int nprops, int per_slot, hipStream_t st) {
     const LinePlan &lp = sh.lp;
     const dim3 block(2 * lp.P * W);
-    switch (lp.base + (lp.rem ? 1 : 0)) {
+    // two lines a block have 32 chunks or more, on lines of over 96 points: chunks of over 3
+    const int steps = lp.base + (lp.rem ? 1 : 0);
+    if (W == 2 && steps < 4) throw std::runtime_error("line walk: unsupported chunk length");
+    switch (steps) {
 #define NMK_STEPS(S)                                                                                                   \
     case S:                                                                                                            \
-        hipLaunchKernelGGL((k_walk<S, W, NEU>), grid, block, 0, st, src, dst, accin, acc, wm, axis, flip, g, sp, pp, \
-                           lp, nprops, per_slot);                                                                      \
+        if constexpr (W > 2 || S > 3)                                                                                  \
+            hipLaunchKernelGGL((k_walk<S, W, NEU>), grid, block, 0, st, src, dst, accin, acc, wm, axis, flip, g, sp, \
+                               pp, lp, nprops, per_slot);                                                              \
         break;
         NMK_STEPS(2)
         NMK_STEPS(3)

@@ -4,6 +4,7 @@ ones on stored stencils elsewhere.  The library runs on the stand-in for the
 HIP runtime (hip_stub/hip_stub.c), which notes the kernels launched."""
 import json
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -54,8 +55,10 @@ stub = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
 stub.stub_name.restype = ctypes.c_char_p
 sys.path.insert(0, sys.argv[2])
 import numpy as np
-from nemaktis_amd import bpm_backend, fields
+from nemaktis_amd import _lib, bpm_backend, fields
 
+_lib.load()
+print("holds", json.dumps([stub.stub_name(i).decode() for i in range(stub.stub_kernels())]))
 for (nx, ny), nq, nwl, precision, _ in json.loads(sys.argv[3]):
     dims = (nx, ny, 2)
     s = fields.make_settings(dims, (0.1, 0.1, 0.1), [0.5 + 0.01 * k for k in range(nwl)],
@@ -70,11 +73,12 @@ for (nx, ny), nq, nwl, precision, _ in json.loads(sys.argv[3]):
 
 
 def launched(so, jobs):
-    """The mangled names of the kernels that each job launches."""
+    """The mangled names of the library's kernels, and of those that each job launches."""
     r = subprocess.run([sys.executable, "-c", DRIVER, so, ROOT, json.dumps(jobs)], stdout=subprocess.PIPE,
                        stderr=subprocess.STDOUT, text=True, timeout=600)
     assert r.returncode == 0, r.stdout[-3000:]
-    return [json.loads(line[6:]) for line in r.stdout.splitlines() if line.startswith("route ")]
+    lines = [line.split(" ", 1) for line in r.stdout.splitlines()]
+    return json.loads(lines[0][1]), [json.loads(v) for k, v in lines if k == "route"]
 
 
 @pytest.fixture(scope="module")
@@ -89,9 +93,19 @@ def stub(tmp_path_factory):
 
 def test_routes(stub):
     got = []
-    for job, names in zip(ROUTES, launched(stub, ROUTES)):
+    for job, names in zip(ROUTES, launched(stub, ROUTES)[1]):
         walks = any("k_walk" in n for n in names)
         stored = any("k_xsolve" in n or "k_ysolve" in n for n in names)
         assert walks != stored, (job, names)
         got.append(job[:4] + (walks,))
     assert got == ROUTES
+
+
+def test_the_library_holds_no_walking_kernel_that_nothing_reaches(stub):
+    holds = launched(stub, [])[0]
+    # FP64 only: the slab material and the kernels of a state with x slow
+    x_slow = r"k_(init_fields|pack_fields|boundary|boundary_point|output|bulk_plane)I%sLb1E"
+    assert not [n for n in holds if re.search("k_slab_materialIf|" + x_slow % "f", n)]
+    assert len([n for n in holds if re.search("k_slab_materialId|" + x_slow % "d", n)]) == 7
+    # two lines a block have chunks of more than 3 points
+    assert not [n for n in holds if re.search(r"k_walkILi[23]ELi2E", n)]
