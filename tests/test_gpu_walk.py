@@ -44,9 +44,8 @@ def _compare(dims, lc, s, mask=None, formula="", E_in=None, **kw):
     assert err.max() < TOL, err.max()
 
 
-# march lines of Nx - 1 and Ny - 1 points: the shortest (16) and longest (1024) with a launch shape and their outer
-# neighbours, every chunk length 2..8 with and without shorter chunks, each lines-per-block (2 above 512 points), last
-# strips of one line
+# march lines of Nx - 1 and Ny - 1 points around the ends of the launch shapes, with last strips of one line; strips that
+# are long along x, and lines above 1024 points, take the stored stencils on both sides
 @pytest.mark.parametrize("Nx,Ny", [(17, 17), (18, 33), (16, 40), (40, 16), (34, 130), (129, 66), (200, 97), (258, 50),
                                    (400, 19), (512, 18), (513, 20), (514, 21), (25, 769), (1024, 17), (18, 1025),
                                    (1026, 17)])
@@ -115,3 +114,20 @@ def test_no_further_from_the_oracle_than_the_stored_stencils(dims):
     walk = bpm_backend.propagate(js, lc)
     stored = bpm_backend.propagate(js, lc, tuning={"x_chunks": 64, "x_rows": 1, "y_chunks": 64, "y_cols": 2})
     assert np.linalg.norm(walk - want) < 1.5 * np.linalg.norm(stored - want)
+
+
+# mesh, directions a wavelength, wavelengths: every kernel instance of the walk (chunks of 2 to 8 points with 16, 8, 4 and 2
+# lines a block) along x and along y, of whole chunks or with shorter ones (tests/test_walk_route_host.py looks them up)
+SHAPES = [(9, 9, 1, 1), (10, 10, 1, 1), (14, 14, 1, 1), (17, 17, 1, 1), (18, 18, 1, 1), (26, 26, 1, 1), (33, 33, 1, 1),
+          (34, 34, 1, 1), (50, 50, 1, 1), (66, 66, 1, 1), (82, 82, 1, 1), (98, 98, 1, 1), (130, 130, 1, 1),
+          (162, 162, 1, 1), (82, 82, 7, 1), (66, 66, 19, 1), (66, 770, 1, 1), (770, 66, 1, 1), (9, 898, 1, 1),
+          (898, 65, 1, 1), (86, 386, 1, 3), (386, 86, 1, 3), (98, 450, 1, 3), (450, 98, 1, 3), (114, 338, 1, 3),
+          (338, 114, 1, 3), (194, 194, 1, 3), (226, 226, 1, 3), (1025, 65, 1, 1), (66, 1024, 1, 1)]
+
+
+@pytest.mark.parametrize("Nx,Ny,nq,nwl", SHAPES)
+def test_every_kernel_instance(Nx, Ny, nq, nwl):
+    dims = (Nx, Ny, 3)
+    s = fields.make_settings(dims, (0.1, 0.13, 0.1), [0.5 + 0.06 * k for k in range(nwl)],
+                             wavevectors=[(0.11 - 0.01 * k, 0.02 * k - 0.07) for k in range(nq)], nhost="1.5")
+    _compare(dims, _director(dims, Nx + Ny), s, wl_batch=0)

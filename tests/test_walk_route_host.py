@@ -109,3 +109,17 @@ def test_the_library_holds_no_walking_kernel_that_nothing_reaches(stub):
     assert len([n for n in holds if re.search("k_slab_materialId|" + x_slow % "d", n)]) == 7
     # two lines a block have chunks of more than 3 points
     assert not [n for n in holds if re.search(r"k_walkILi[23]ELi2E", n)]
+
+
+def test_gpu_tests_cover_every_instance(stub):
+    """k_walk's instances in the jobs of test_gpu_walk.test_every_kernel_instance."""
+    from test_gpu_walk import SHAPES
+
+    holds, runs = launched(stub, [((nx, ny), nq, nwl, 64, True) for nx, ny, nq, nwl in SHAPES])
+    instance = re.compile(r"k_walkILi\d+ELi\d+ELi[01]E")
+    found = set()
+    for (nx, ny, nq, nwl), names in zip(SHAPES, runs):
+        got = {m.group() for m in map(instance.search, names) if m}
+        assert got, "%d x %d does not walk" % (nx, ny)
+        found |= got
+    assert found == {m.group() for m in map(instance.search, holds) if m}
