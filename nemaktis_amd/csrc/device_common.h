@@ -100,16 +100,14 @@ struct SlotParams {
     double alpha_im;      // absorption factor alpha = 1 + i*alpha_im
     double nin, nout_fresnel, nout_filter;
     double nref;          // filled on the device by the reduction
-    // factors of the mu*R stencils (R = (D S^-1 + S^-1 D)/4 + i W, mu = i dZ/2): (dZ/8) times 1/dX^2, 1/dY^2 and
-    // 1/(4 dX dY), and dZ/2 times 1/(8 dX), 1/(8 dY)
-    double rx2, ry2, rxy, gx, gy;
     int iwl;              // wavelength index in the caller's array
     int pad;
 };
 
 // per-propagation (wavelength slot, wavevector, polarisation) scalars
 struct PropParams {
-    int slot, iq, pol, pad;
+    int slot, iq, pol;
+    int iwl;              // wavelength index in the caller's array
     int ox, oy;           // first tap offset of the Catmull-Rom shift (floor(s)-1)
     double wx[4], wy[4];  // Catmull-Rom weights along x and y
     int o1x, o1y, o2x, o2y;      // first tap of one shift / of two composed shifts

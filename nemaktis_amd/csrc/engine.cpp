@@ -311,6 +311,7 @@ public:
             }
             HIPCHK(hipMemcpyAsync(d.ptr, h.data(), d.bytes(), hipMemcpyHostToDevice, st_));
         };
+        upload_steps();
         twiddles(p.Nx, twx_, htwx_);
         twiddles(p.Ny, twy_, htwy_);
         HIPCHK(hipStreamSynchronize(st_));
@@ -448,23 +449,27 @@ private:
     DevBuf<SlotParams> sp_;
     DevBuf<PropParams> pp_;
     // values of the line solvers' buffers: stored stencils and x-line rows, or
-    // (walking solvers) the slab material in both axis orders and the phase
-    // operators beside it
+    // (walking solvers) the slab material in both axis orders, the phase
+    // operators beside it and the stencils' factors of every wavelength
     struct SolverCounts {
-        size_t cf = 0, xt = 0, mat = 0, phase = 0;
+        size_t cf = 0, xt = 0, mat = 0, phase = 0, steps = 0;
     };
     struct SolverBuffers {
         DevBuf<C2<T>> cf, xt, phase;
         DevBuf<c64> mat;
-        void bind(DeviceAllocator *a) { bind_source(a, cf, xt, phase, mat); }
-        SolverCounts counts() const { return {cf.count, xt.count, mat.count, phase.count}; }
-        size_t footprint() const { return cf.footprint() + xt.footprint() + mat.footprint() + phase.footprint(); }
+        DevBuf<WalkSteps> steps;
+        void bind(DeviceAllocator *a) { bind_source(a, cf, xt, phase, mat, steps); }
+        SolverCounts counts() const { return {cf.count, xt.count, mat.count, phase.count, steps.count}; }
+        size_t footprint() const {
+            return cf.footprint() + xt.footprint() + mat.footprint() + phase.footprint() + steps.footprint();
+        }
         // buffers of at least n values wherever o has fewer
         void alloc_beside(const SolverBuffers &o, const SolverCounts &n) {
             if (n.cf > o.cf.count) cf.alloc(n.cf);
             if (n.xt > o.xt.count) xt.alloc(n.xt);
             if (n.mat > o.mat.count) mat.alloc(n.mat);
             if (n.phase > o.phase.count) phase.alloc(n.phase);
+            if (n.steps > o.steps.count) steps.alloc(n.steps);
         }
         // takes over what `fresh` holds and gives back what n leaves out
         void adopt(SolverBuffers &fresh, const SolverCounts &n) {
@@ -476,6 +481,7 @@ private:
             one(xt, fresh.xt, n.xt);
             one(mat, fresh.mat, n.mat);
             one(phase, fresh.phase, n.phase);
+            one(steps, fresh.steps, n.steps);
         }
     };
     SolverBuffers solver_;
@@ -495,6 +501,7 @@ private:
     LinePlan lpx_{}, lpy_{};
     Tuning tune_{};
     std::vector<SlotParams> hsp_;
+    std::vector<WalkSteps> hsteps_;
     std::vector<PropParams> hpp_;
     bool unshifted_[3] = {false, false, false};  // by number of shifts of a boundary
     std::vector<hipEvent_t> evs_;
@@ -549,6 +556,27 @@ private:
         prof_fam_.clear();
     }
 
+    // mesh spacings in units of the wavelength
+    void set_spacings(SlotParams &sp, int w) const {
+        sp.k0 = 2 * kPi / p_.wl[w];
+        sp.dX = sp.k0 * p_.dx;
+        sp.dY = sp.k0 * p_.dy;
+        sp.dZ = sp.k0 * p_.dz;
+    }
+
+    // the factors that the walking solvers read, once their buffers are there (again)
+    void upload_steps() {
+        if (!walk_ || !solver_ready_) return;
+        hsteps_.resize(sz_.nwl);
+        for (int w = 0; w < sz_.nwl; w++) {
+            SlotParams sp;
+            set_spacings(sp, w);
+            hsteps_[w] = {0.125 * sp.dZ / (sp.dX * sp.dX), 0.125 * sp.dZ / (sp.dY * sp.dY),
+                          0.03125 * sp.dZ / (sp.dX * sp.dY), 0.0625 * sp.dZ / sp.dX, 0.0625 * sp.dZ / sp.dY};
+        }
+        HIPCHK(hipMemcpyAsync(solver_.steps.ptr, hsteps_.data(), sz_.nwl * sizeof(WalkSteps), hipMemcpyHostToDevice, st_));
+    }
+
     void setup_batch(int w0, int nslots, int nprops) {
         const Problem &p = p_;
         hsp_.assign(nslots, SlotParams());
@@ -556,10 +584,7 @@ private:
             const int w = w0 + s;
             SlotParams &sp = hsp_[s];
             std::memset(&sp, 0, sizeof(sp));
-            sp.k0 = 2 * kPi / p.wl[w];
-            sp.dX = sp.k0 * p.dx;
-            sp.dY = sp.k0 * p.dy;
-            sp.dZ = sp.k0 * p.dz;
+            set_spacings(sp, w);
             sp.no = p.no[w];
             sp.ne = p.ne[w];
             sp.ne_imag = p.ne_imag[w];
@@ -568,11 +593,6 @@ private:
             sp.ea = sp.ne * sp.ne - sp.eperp;
             sp.ehost = sp.nhost * sp.nhost;
             sp.alpha_im = p.ne_imag[w] / (p.ne[w] - p.no[w]);  // NaN/inf when ne == no, as the reference
-            sp.rx2 = 0.125 * sp.dZ / (sp.dX * sp.dX);
-            sp.ry2 = 0.125 * sp.dZ / (sp.dY * sp.dY);
-            sp.rxy = 0.03125 * sp.dZ / (sp.dX * sp.dY);
-            sp.gx = 0.0625 * sp.dZ / sp.dX;
-            sp.gy = 0.0625 * sp.dZ / sp.dY;
             sp.nin = p.nin[w];
             sp.nout_fresnel = p.nout_fresnel[w];
             sp.nout_filter = p.nout[w];
@@ -597,6 +617,7 @@ private:
                     pp.slot = s;
                     pp.iq = iq;
                     pp.pol = pol;
+                    pp.iwl = w0 + s;
                     pp.qx = qx;
                     pp.qy = qy;
                     const double th = 0.5 * kPi * pol;
@@ -861,6 +882,7 @@ private:
             WalkMaterial wm;
             wm.nat = ring.mat + b * ring.mat_stride;
             wm.tr = wm.nat + (size_t)nslots * walk_points(g_.Mx, g_.My) * 5;
+            wm.steps = solver_.steps.ptr;
             C2<T> *in = cur;
             for (int axis = 0; axis < 2; axis++) {
                 const WalkShape &sh = axis == 0 ? wx_ : wy_;
@@ -870,14 +892,14 @@ private:
                 C2<T> *done = nw > 0 ? cur : axis == 0 ? other : cur;
                 timed(fam, [&] {
                     launch_walk(axis, 0, in, nw > 0 ? A : nullptr, nullptr, nw > 0 ? nullptr : done, nw == 0, wm, g_,
-                                sp_.ptr, pp_.ptr, nprops, 2 * sz_.nq, sh, st_);
+                                pp_.ptr, nprops, 2 * sz_.nq, sh, st_);
                 });
                 C2<T> *a = A, *bb = B;
                 for (int it = 0; it < nw; it++) {
                     const bool last = it + 1 == nw;
                     timed(fam, [&] {
                         launch_walk(axis, 1, a, last ? nullptr : bb, it == 0 ? a : other, last ? done : other, last, wm,
-                                    g_, sp_.ptr, pp_.ptr, nprops, 2 * sz_.nq, sh, st_);
+                                    g_, pp_.ptr, nprops, 2 * sz_.nq, sh, st_);
                     });
                     std::swap(a, bb);
                 }
@@ -917,6 +939,7 @@ private:
             SolverCounts n;
             n.mat = (size_t)sz_.ring * mat_slab();
             n.phase = (size_t)sz_.ring * sz_.nslots_max * 3 * sz_.NP;
+            n.steps = sz_.nwl;
             hold_buffers(n);
             walk_ = true;
             wx_ = wx;
@@ -987,7 +1010,13 @@ private:
     void retune(const Tuning &t) override {
         HIPCHK(hipStreamSynchronize(st_));
         if (st2_) HIPCHK(hipStreamSynchronize(st2_));
-        set_tuning(t);
+        try {
+            set_tuning(t);
+        } catch (...) {
+            upload_steps();  // (the buffers may have been taken anew)
+            throw;
+        }
+        upload_steps();
     }
 
     void output_batch(int w0, int nslots, int nprops, const C2<T> *state) {

@@ -469,8 +469,7 @@ __device__ __forceinline__ void walk_lines(int tid, const LinePlan &lp, const c6
 template <int STEPS, int W, int NEU>
 __global__ __launch_bounds__(512) void k_walk(const c64 *__restrict__ src, c64 *__restrict__ dst,
                                               const c64 *accin, c64 *acc, WalkMaterial wm, int axis, int flip,
-                                              Geo g, const SlotParams *__restrict__ sp,
-                                              const PropParams *__restrict__ pp, LinePlan lp, int nprops,
+                                              Geo g, const PropParams *__restrict__ pp, LinePlan lp, int nprops,
                                               int per_slot) {
     using C = c64;
     using R = Stage<W>;
@@ -495,7 +494,7 @@ __global__ __launch_bounds__(512) void k_walk(const c64 *__restrict__ src, c64 *
     const bool active = t < Mt;
 
     const int slot = pp[prop].slot;
-    const SlotParams &s = sp[slot];
+    const WalkSteps &s = wm.steps[pp[prop].iwl];
     Steps st;
     st.l2 = axis == 0 ? s.rx2 : s.ry2;
     st.t2 = axis == 0 ? s.ry2 : s.rx2;
@@ -639,8 +638,8 @@ __global__ __launch_bounds__(512) void k_walk(const c64 *__restrict__ src, c64 *
 
 template <int W, int NEU>
 static void walk_dispatch(const WalkShape &sh, dim3 grid, const c64 *src, c64 *dst, const c64 *accin, c64 *acc,
-                          const WalkMaterial &wm, int axis, int flip, const Geo &g, const SlotParams *sp,
-                          const PropParams *pp, int nprops, int per_slot, hipStream_t st) {
+                          const WalkMaterial &wm, int axis, int flip, const Geo &g, const PropParams *pp,
+                          int nprops, int per_slot, hipStream_t st) {
     const LinePlan &lp = sh.lp;
     const dim3 block(2 * lp.P * W);
     // two lines a block have 32 chunks or more, on lines of over 96 points: chunks of over 3
@@ -650,8 +649,8 @@ static void walk_dispatch(const WalkShape &sh, dim3 grid, const c64 *src, c64 *d
 #define NMK_STEPS(S)                                                                                                   \
     case S:                                                                                                            \
         if constexpr (W > 2 || S > 3)                                                                                  \
-            hipLaunchKernelGGL((k_walk<S, W, NEU>), grid, block, 0, st, src, dst, accin, acc, wm, axis, flip, g, sp, \
-                               pp, lp, nprops, per_slot);                                                              \
+            hipLaunchKernelGGL((k_walk<S, W, NEU>), grid, block, 0, st, src, dst, accin, acc, wm, axis, flip, g, pp, \
+                               lp, nprops, per_slot);                                                              \
         break;
         NMK_STEPS(2)
         NMK_STEPS(3)
@@ -667,8 +666,8 @@ static void walk_dispatch(const WalkShape &sh, dim3 grid, const c64 *src, c64 *d
 }
 
 void launch_walk(int axis, int neumann, const c64 *src, c64 *dst, const c64 *accin, c64 *acc, bool flip,
-                 const WalkMaterial &wm, const Geo &g, const SlotParams *sp, const PropParams *pp, int nprops,
-                 int per_slot, const WalkShape &sh, hipStream_t st) {
+                 const WalkMaterial &wm, const Geo &g, const PropParams *pp, int nprops, int per_slot,
+                 const WalkShape &sh, hipStream_t st) {
     const LinePlan &lp = sh.lp;
     const int Ml = axis == 0 ? g.Mx : g.My, Mt = axis == 0 ? g.My : g.Mx;
     // a wave holds chunks of one component; rows and result of a block fit its LDS buffers; the reduction takes a stage
@@ -680,8 +679,8 @@ void launch_walk(int axis, int neumann, const c64 *src, c64 *dst, const c64 *acc
     const dim3 grid((unsigned)((items + 7) / 8 * 8));
 #define NMK_WALK(WW)                                                                                                    \
     if (sh.W == WW) {                                                                                                   \
-        if (neumann) walk_dispatch<WW, 1>(sh, grid, src, dst, accin, acc, wm, axis, flip, g, sp, pp, nprops, per_slot, st); \
-        else walk_dispatch<WW, 0>(sh, grid, src, dst, accin, acc, wm, axis, flip, g, sp, pp, nprops, per_slot, st);         \
+        if (neumann) walk_dispatch<WW, 1>(sh, grid, src, dst, accin, acc, wm, axis, flip, g, pp, nprops, per_slot, st); \
+        else walk_dispatch<WW, 0>(sh, grid, src, dst, accin, acc, wm, axis, flip, g, pp, nprops, per_slot, st);         \
         return;                                                                                                         \
     }
     NMK_WALK(16)

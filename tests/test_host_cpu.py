@@ -190,6 +190,19 @@ def test_footprint_estimate_scales():
     assert 512 * 512 * 100 * 24 < out.value < b64
 
 
+# bytes of device memory that a job has always been admitted with (three wavelengths marched together)
+@pytest.mark.parametrize("n,precision,want", [(33, 32, 9217024), (33, 64, 18064384), (161, 32, 67841024),
+                                              (161, 64, 127560704)])
+def test_footprint_of_a_job_does_not_grow(n, precision, want):
+    lib = _lib.load()
+    s = fields.make_settings((n, n, 5), (0.1,) * 3, [0.5, 0.51, 0.52])
+    out, err = ctypes.c_int64(), _lib.err_buf()
+    o = _lib.options(precision=precision, wl_batch=0)
+    assert lib.nmk_bpm_estimate_footprint(json.dumps(s).encode(), n * n * 5 * 3, 0, ctypes.byref(o),
+                                          ctypes.byref(out), err, len(err)) == 0
+    assert out.value <= want
+
+
 @pytest.mark.parametrize("expr,lam", [("1.7+0.01/lambda^2", 0.55), ("-2^2", 0.6), ("2^3^2", 0.6),
                                       ("1.5-0.003/lambda^2+sqrt(lambda)", 0.45)])
 def test_oracle_expression_evaluator_agrees_with_backend(expr, lam):

@@ -63,7 +63,7 @@ with context(first) as c:
     assert marches(c) == want
     c.set_tuning(first)
     assert marches(c) == own and stub.stub_live() == held
-assert stub.stub_live() == 0
+assert stub.stub_live() == 0 and stub.stub_unfit() == 0
 print("refused" if refused else "switched", "lost" if lost else "kept")
 """
 
