@@ -70,8 +70,13 @@ def algorithmic_bytes(fam, c, nprops, nslots, NP, Nfull, fd, nw):
     return None
 
 
-# the FP64 march at the built-in shapes (mesh axes of 17 to 1025 points): solvers that generate their stencils
+# the FP64 march of this benchmark's 512^2 job at the built-in shapes: solvers that generate their stencils
 KERNELS_WALK = {"solve_x": "k_walk", "solve_y": "k_walk", "boundary": "k_boundary", "coefs": "k_slab_material"}
+
+
+def walks(precision, tuning):
+    """Whether the 512^2 job marches so (other meshes and batches go by a rule of the library's own)."""
+    return precision == 64 and tuning is None
 
 
 def walk_bytes(fam, nprops, nslots, NP, Nfull, fd, nw):
@@ -480,7 +485,7 @@ def drop_in_masked_leg():
 
 
 def roofline_of(js, lc, n_E, precision, wl_batch, steps, Nx, Ny, nprops, nq, fd, nw, tuning=None):
-    """Dominant march kernel family of the path, its average launch time
+    """Dominant march kernel family of the path of a 512^2 job, its average launch time
     (HIP events on its launch stream, eager), and its bandwidth two ways:
     the workload's algorithmic bytes per voxel-slice update (64 / 128 B of
     field traffic + 24 B of director per slot, shared by the slot's 2 Nq
@@ -496,7 +501,7 @@ def roofline_of(js, lc, n_E, precision, wl_batch, steps, Nx, Ny, nprops, nq, fd,
     algo = per_update * units
     achieved = algo / (avg_ms * 1e-3) / 1e9
     c = 8 if precision == 32 else 16
-    walk = precision == 64 and tuning is None and 17 <= min(Nx, Ny) and max(Nx, Ny) <= 1025
+    walk = walks(precision, tuning)
     if walk:
         local = walk_bytes(dom, nprops, nprops // (2 * nq), (Nx - 1) * (Ny - 1), Nx * Ny, fd, nw)
     else:

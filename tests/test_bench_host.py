@@ -37,5 +37,19 @@ def test_byte_model_of_the_march_kernels_matches_the_hbm_counters(precision):
         assert 0.98 <= measured / model <= 1.15, (kernel, measured / model)
 
 
+def test_byte_model_of_the_walking_solvers_matches_the_hbm_counters():
+    """The same job at the built-in shapes.  The walk's blocks hold 4 lines and
+    read material and source on two columns more, half as much again, as far
+    as that misses the caches: 80 + 64 of the 251 bytes a point, so at most
+    1.29 times the model."""
+    path = os.path.join(ROOT, "profiles", "hbm_traffic_random512_fp64_walk.txt")
+    for fam, kernel, most in (("solve_x", "k_walk", 1.29), ("solve_y", "k_walk", 1.29),
+                              ("boundary", "k_boundary_point", 1.15), ("coefs", "k_slab_material", 1.15)):
+        measured, src = bench.measured_traffic(kernel, path)
+        assert measured is not None and src.startswith("profiles"), kernel
+        model = bench.walk_bytes(fam, 2, 1, 511 * 511, 512 * 512, 3, 2)
+        assert 0.98 <= measured / model <= most, (kernel, measured / model)
+
+
 def test_missing_traffic_summary_gives_none():
     assert bench.measured_traffic("k_ysolve", os.path.join(ROOT, "profiles", "no_such_file.txt")) == (None, None)

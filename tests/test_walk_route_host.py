@@ -123,3 +123,13 @@ def test_gpu_tests_cover_every_instance(stub):
         assert got, "%d x %d does not walk" % (nx, ny)
         found |= got
     assert found == {m.group() for m in map(instance.search, holds) if m}
+
+
+def test_bench_names_the_kernels_of_its_512_job(stub):
+    sys.path.insert(0, ROOT)
+    import bench
+
+    for precision in (64, 32):
+        names = " ".join(launched(stub, [((512, 512), 1, 1, precision, True)])[1][0])
+        named = bench.KERNELS_WALK if bench.walks(precision, None) else bench.KERNELS
+        assert all(named[fam] in names for fam in ("solve_x", "solve_y", "boundary", "coefs"))
