@@ -110,7 +110,8 @@ __device__ __forceinline__ void fft_stage(const c64 *__restrict__ b0, c64 *__res
                 c64 a = u[0], e = mk(0.0, 0.0);
 #pragma unroll
                 for (int q = 1; q <= H; q++) {
-                    const c64 w = wr[(k1 * q) % R];
+                    const int m = (k1 * q) % R;  // (the second half mirrors the first: fewer registers)
+                    const c64 w = m <= H ? wr[m] : conj(wr[R - m]);
                     a = mk(fma(u[q].x, w.x, a.x), fma(u[q].y, w.x, a.y));
                     e = mk(fma(u[R - q].x, w.y, e.x), fma(u[R - q].y, w.y, e.y));
                 }
