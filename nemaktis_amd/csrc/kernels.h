@@ -149,6 +149,9 @@ struct FftPlan {
     int direct;
 };
 FftPlan make_fft_plan(int n);
+// whether a pass over `lines` lines of the plan goes by the direct sum (across: adjacent columns of a plane)
+enum class FftPass { rows, columns, refocus };
+bool fft_direct(const FftPlan &pl, FftPass pass, int64_t lines, int across);
 // unnormalised DFT of lines of length n, sign -1 forward, +1 backward, with
 // the twiddle table tw[m] = exp(-2 pi i m / n): `lines` lines per plane, line
 // i of plane p starting at p*plane_size + i*line_stride, elements elem_stride

@@ -2576,6 +2576,39 @@ FftPlan make_fft_plan(int n) {
     return pl;
 }
 
+// Stages of primes above 13 pay when a launch has enough lines to fill their
+// eight-column matrix tiles and the device; the direct sum spreads every output
+// over a thread and wins below.  Direct / staged us, one launch:
+//   rows: 64 lines of 127 points 6.7 / 13, 4096 33 / 15; of 509 37 / 65, at 1024
+// 113 / 65; of 161 7.9 / 8.2, at 512 10.8 / 8.6; a prime length above 1024, two
+// lines a block and a quarter of a tile, 1201 points 197 / 359, at 16384 9170 / 11600
+//   columns: 17 points, 16384 lines, 5.9 / 11; a prime above 1024, 1409 points 278 /
+// 487 (1301 points 439 / 410, at 1024 lines slower too); else 1.1 to 14 times as
+// fast as the direct sum
+//   refocus columns, whose staged form fuses two transforms and the filter: 1.2 to
+// 20 times, but for 64 lines of 1409 points 557 / 626 (1301 880 / 543; 1409 at 512
+// lines 932 / 640) and 17 points at 16384 lines 16.8 / 17.9
+// across: adjacent columns of a plane; below 8 a staged block is partly padding
+// (16384 columns of 23 points, four a plane: 0.70 times)
+bool fft_direct(const FftPlan &pl, FftPass pass, int64_t lines, int across) {
+    if (pl.direct) return true;
+    if (fft_mode(pl) != FFT_ANY) return false;
+    const int n = pl.n;
+    const bool prime = pl.big[0] == n;
+    switch (pass) {
+    case FftPass::rows:
+        if (n < 64) return lines < 4096;
+        if (n < 128) return lines < 2048;
+        if (prime) return n > 1024 || lines < 1024;
+        return n < 256 && lines < 512;
+    case FftPass::columns:
+        return n < 32 || (n < 40 && lines > 8192) || (prime && n > 1024);
+    default:
+        if (prime && n > 1365 && lines < 512) return true;
+        return (n < 20 && lines > 8192) || (n < 48 && across < 8 && lines > 2048);
+    }
+}
+
 // rows: block b transforms lines C*b .. C*b+C-1 of the whole batch (each a
 // contiguous run of n values); src and dst may be the same buffer.  A fourth wave
 // per SIMD: at 132 registers 16384 lines of 640 points took 165 us, at 127 141, at
@@ -2621,7 +2654,7 @@ __global__ __launch_bounds__(256) void k_fft_cols(c64 *__restrict__ data, int Nx
     }
 }
 
-// Direct DFT of lines (above 2048 points): a block holds C
+// Direct DFT of lines (above 2048 points, or where fft_direct has it): a block holds C
 // lines and the twiddle table in LDS; output k of a line is
 // sum_j x_j tw[(j k) mod n] (conjugated twiddles for sign +1), with the twiddle
 // index advanced by k per term (no products or divisions in the loop).
@@ -2676,7 +2709,7 @@ void launch_dft_lines(const c64 *src, c64 *dst, int n, int lines, int planes, in
 
 void launch_fft_rows(const c64 *src, c64 *dst, int Nx, int Ny, int planes, int sign, const c64 *tw_x,
                      const FftPlan &px, hipStream_t st) {
-    if (px.direct) {
+    if (fft_direct(px, FftPass::rows, (int64_t)Ny * planes, Nx)) {
         launch_dft_lines(src, dst, Nx, Ny, planes, (int64_t)Nx * Ny, Nx, 1, sign, tw_x, st);
         return;
     }
@@ -2693,7 +2726,8 @@ void launch_fft_rows(const c64 *src, c64 *dst, int Nx, int Ny, int planes, int s
     case CC:                                                      \
         if (mode == FFT_POW2) launch(k_fft_rows<CC, FFT_POW2>);   \
         else if (mode == FFT_SMALL) launch(k_fft_rows<CC, FFT_SMALL>); \
-        else launch(k_fft_rows<CC, FFT_ANY>);                     \
+        else if constexpr (CC > 1) launch(k_fft_rows<CC, FFT_ANY>); \
+        else throw std::runtime_error("transform: bad block shape"); \
         break;
         NMK_ROWS(16)
         NMK_ROWS(8)
@@ -2708,7 +2742,7 @@ void launch_fft_rows(const c64 *src, c64 *dst, int Nx, int Ny, int planes, int s
 
 void launch_fft_cols(c64 *data, int Nx, int Ny, int planes, int sign, const c64 *tw_y, const FftPlan &py,
                      hipStream_t st) {
-    if (py.direct) {
+    if (fft_direct(py, FftPass::columns, (int64_t)Nx * planes, Nx)) {
         launch_dft_lines(data, data, Ny, Nx, planes, (int64_t)Nx * Ny, 1, Nx, sign, tw_y, st);
         return;
     }
@@ -2726,7 +2760,8 @@ void launch_fft_cols(c64 *data, int Nx, int Ny, int planes, int sign, const c64 
     case CC:                                                      \
         if (mode == FFT_POW2) launch(k_fft_cols<CC, FFT_POW2>);   \
         else if (mode == FFT_SMALL) launch(k_fft_cols<CC, FFT_SMALL>); \
-        else launch(k_fft_cols<CC, FFT_ANY>);                     \
+        else if constexpr (CC > 1) launch(k_fft_cols<CC, FFT_ANY>); \
+        else throw std::runtime_error("transform: bad block shape"); \
         break;
         NMK_COLS(8)
         NMK_COLS(4)

@@ -130,7 +130,7 @@ __global__ __launch_bounds__(NT, MODE == FFT_ANY ? 3 : 1) void k_view_columns(c6
 }
 
 // fields of the 4 components of every (wavelength, wavevector) times its
-// filter plane (the column pass of lengths without an LDS plan)
+// filter plane (the column pass by the direct sum)
 __global__ __launch_bounds__(256) void k_view_apply_filter(c64 *__restrict__ data, const c64 *__restrict__ filt,
                                                            int64_t N) {
     const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -141,7 +141,7 @@ __global__ __launch_bounds__(256) void k_view_apply_filter(c64 *__restrict__ dat
 
 void launch_view_columns(c64 *data, const c64 *filt, int Nx, int Ny, int nlq, const c64 *tw_y, const FftPlan &py,
                          hipStream_t st) {
-    if (py.direct) {
+    if (fft_direct(py, FftPass::refocus, (int64_t)Nx * nlq * 4, Nx)) {
         // direct DFT of the columns, the filter, and the inverse DFT
         const int64_t N = (int64_t)Nx * Ny;
         launch_dft_lines(data, data, Ny, Nx, nlq * 4, N, 1, Nx, -1, tw_y, st);
@@ -174,7 +174,8 @@ void launch_view_columns(c64 *data, const c64 *filt, int Nx, int Ny, int nlq, co
     case CC:                                                               \
         if (mode == FFT_POW2) launch(k_view_columns<CC, FFT_POW2>, 256);   \
         else if (mode == FFT_SMALL) launch(k_view_columns<CC, FFT_SMALL>, 256); \
-        else launch(k_view_columns<CC, FFT_ANY>, 256);                     \
+        else if constexpr (CC > 1) launch(k_view_columns<CC, FFT_ANY>, 256); \
+        else throw std::runtime_error("transform: bad block shape"); \
         break;
         NMK_VCOLS(8)
         NMK_VCOLS(4)
