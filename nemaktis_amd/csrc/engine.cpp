@@ -184,7 +184,7 @@ WalkShape walk_shape(int M, int Mt, int nprops) {
 }
 
 // Whether a march of nprops propagations, nq directions a wavelength, is
-// faster with the walking solvers than on stored stencils (850 meshes and
+// faster with the walking solvers than on stored stencils (1100 meshes and
 // batches of 9 to 1024 points an axis timed both ways, us a slab stored ->
 // walking).  The walk generates the stencils for every propagation, reads two
 // columns beside the lines of a block and two rows beside each chunk, and has
@@ -199,17 +199,22 @@ WalkShape walk_shape(int M, int Mt, int nprops) {
 // 159, 601 x 21 at 7 121 -> 139).
 //   Several directions share: from 128-point y lines (600 x 130 at 7
 // directions 505 -> 479, 1000 x 200 1085 -> 1075; 600 x 64 225 -> 256, 1000 x 12
-// at 37 271 -> 583), and beyond a ring of them only where blocks hold many
-// lines along x and not too many rounds along y (200^2 at 37 981 -> 940, 300 x
-// 600 at 19 2540 -> 2320; 1000 x 300 at 37 9020 -> 10930, 256 x 1000 8210 -> 8520,
-// 64 x 1000 1870 -> 2060, 340 x 600 at 61 12380 -> 13020).
+// at 37 271 -> 583), from 120-point ones beside x lines of medium length (127 x
+// 127 at 7 directions of 21 wavelengths 1411 -> 1215, 380 x 120 of 3 635 -> 531),
+// and from 300-point ones beside the longest at several wavelengths (1000 x 300
+// at 7 of 3 5230 -> 5060; 1000 x 170 2730 -> 2780).
+//   Beyond a ring of directions only where blocks hold many lines along x and
+// not too many rounds along y (200^2 at 37 981 -> 940, 300 x 600 at 19 2540 ->
+// 2320; 1000 x 300 at 37 9020 -> 10930, 256 x 1000 8210 -> 8520, 64 x 1000 1870 ->
+// 2060, 340 x 600 at 61 12380 -> 13020).
 bool walk_pays(int Mx, int My, int nq, int nprops, const WalkShape &wx, const WalkShape &wy) {
     if (wx.W == 0 || wy.W == 0 || Mx > 16 * My) return false;
     auto blocks = [&](const WalkShape &w, int Mt) { return (int64_t)((Mt + w.W - 1) / w.W) * nprops; };
     if (blocks(wx, My) <= 256 && blocks(wy, Mx) <= 256) return true;
     if (nq == 1) return My >= 64;
-    if (nq <= 7) return My >= 128;
-    return My >= 128 && My <= (nq <= 37 ? 640 : 400) && Mx >= 96 && Mx <= 384;
+    const bool medium = Mx >= 96 && Mx <= 384;
+    if (nq <= 7) return My >= (medium ? 120 : Mx <= 860 || nprops == 2 * nq ? 128 : 300);
+    return medium && My >= 128 && My <= (nq <= 37 ? 640 : 400);
 }
 
 template <class T>

@@ -33,6 +33,10 @@ ROUTES = [
     ((1001, 13), 1, 7, 64, False),     # 124 / 163
     ((601, 131), 7, 1, 64, True),      # 505 / 479
     ((1001, 201), 7, 1, 64, True),     # 1085 / 1075
+    ((128, 128), 7, 21, 64, True),     # 1411 / 1215
+    ((1001, 121), 7, 3, 64, False),    # 1715 / 1797
+    ((1001, 171), 7, 3, 64, False),    # 2730 / 2780
+    ((1001, 301), 7, 3, 64, True),     # 5230 / 5060
     ((601, 65), 7, 1, 64, False),      # 225 / 256
     ((301, 41), 7, 1, 64, False),      # 113 / 125
     ((1000, 12), 37, 1, 64, False),    # 271 / 583
