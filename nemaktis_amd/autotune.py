@@ -112,8 +112,9 @@ def cache_key(precision, Nx, Ny, nprops, use_graph=True):
 
 def _time(ctx, tuning, reps):
     """Median march time of the resident job with `tuning` (inf when the
-    device refuses the shape).  One context serves every candidate: buffers
-    that a captured graph has used are never freed between candidates."""
+    device refuses the shape).  One context serves every candidate; only a
+    change between the built-in FP64 solvers and explicit shapes exchanges the
+    solvers' buffers, after the graphs that hold them are gone."""
     try:
         ctx.set_tuning(tuning)
     except bpm_backend.BpmBackendError:
@@ -127,9 +128,8 @@ def _time(ctx, tuning, reps):
 
 def tune(settings, lc_vals, precision=32, wl_batch=0, depth=9, reps=3, use_cache=True, log=None, use_graph=True):
     """Returns the best tuning dict for this job's transverse mesh (None: the
-    built-in shapes), measured
-    on a `depth`-plane copy of it (graph replay or eager launches, as the job
-    will run), plus the timing table."""
+    built-in shapes), measured on a `depth`-plane copy of it (graph replay or
+    eager launches, as the job will run), plus the timing table."""
     ic = settings["Physics settings"]["Initial conditions"]
     Nx, Ny, Nz = ic["Mesh dimensions"]
     co = settings["Physics settings"]["Coefficients"]
@@ -157,7 +157,7 @@ def tune(settings, lc_vals, precision=32, wl_batch=0, depth=9, reps=3, use_cache
     try:
         best, best_ms, table, t0 = _search(ctx, best, xs, ys, Mx, My, precision, reps)
         # the built-in shapes, which in FP64 march with other solvers than explicit ones ask for
-        # (512^2, one pair: 17.5 ms against 25 ms for the best explicit shape)
+        # (512^2, one pair: 17.3 ms against 25 ms for the best explicit shape)
         ms = _time(ctx, None, reps)
         table.append((None, ms))
         if ms <= best_ms:

@@ -157,7 +157,7 @@ int pow2_at_least(int v) {
 // Launch shape of the walking solvers for lines of M points, Mt of them per
 // component and propagation: P chunks of a line and W lines a block, at most
 // 512 threads of both components, whole waves of one component; chunks of at
-// most 8 points (16 spill).  W = 0: no shape (lines over 1024 or under 16
+// most 8 points (16 spill).  W = 0: no shape (lines over 1024 or under 8
 // points).
 //
 // A block is alone on its CU, so up to 256 blocks a launch takes as long as
@@ -1061,7 +1061,9 @@ Tuning default_tuning(int precision, int Mx, int My, int nprops) {
     // after: 256^2 at 147 pairs 3418 -> 3309, 301 x 203 at 21 pairs 631 -> 554,
     // 400 x 300 at 28 pairs 1639 -> 1503, 128^2 at 14 pairs 161 -> 131, 512^2 at
     // 2 pairs 352 -> 314; a lone pair gains up to 400 points (256^2 109 -> 106)
-    // and loses at 512 (188 -> 191)
+    // and loses at 512 (188 -> 191).  Over 120 random meshes and batches the FP32
+    // march is at least 0.993 times as fast as with the shapes before; its error
+    // against FP64, over 91 outputs of 47 jobs that changed shape, 0.98 times
     const int longest = std::max(Mx, My);
     const bool lean = precision == 32 && longest <= 512 && (nprops > 2 || longest <= 400);
     const int lcap = precision == 32 && !lean ? 16 : 8;

@@ -131,8 +131,8 @@ __device__ __forceinline__ void fft_stage(const c64 *__restrict__ b0, c64 *__res
 // columns, four terms q a step): a column is the real or imaginary part of one
 // butterfly, so that neither operand needs more than one LDS word per lane and
 // step.  Waves take the tiles in turn; rows past R / 2 and terms past it are
-// padding.  161 points (7 x 23), 532 planes of 161 lines: rows 158 us and the
-// refocus columns 278 us a pass, where the direct sum over the whole length
+// padding.  161 points (7 x 23), 532 planes of 161 lines: rows 144-180 us and the
+// refocus columns 280 us a pass, where the direct sum over the whole length
 // took 844 us for each of their transforms; the bound is latency (two blocks
 // of waves a CU, a barrier between the short stages), not the matrix cores,
 // busy about a tenth of it.

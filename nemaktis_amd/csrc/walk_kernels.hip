@@ -19,9 +19,9 @@
 //
 // What bounds it: at one propagation pair on 512^2 two waves per SIMD, one of
 // each component, FP64 arithmetic about half of the time (200 instructions a
-// row of the two) and 69-86 MB of traffic a launch; at 64^2 the chain of steps
+// row of the two) and 81 MB of traffic a launch; at 64^2 the chain of steps
 // and cyclic reductions.  Device time per launch, MI355X, against the solvers
-// on stored stencils (x / y lines): 512^2 x 1 pair 22-23 us (29-36 / 34-36),
+// on stored stencils (x / y lines): 512^2 x 1 pair 22-23 us (29-36 / 35),
 // 1024^2 120-125 us (130-156 / 225-238).  Per slab, whole march: 64^2 54 us
 // (68), 161^2 74 us (96), 128^2 x 7 pairs 109 us (120), x 147 pairs 1.27 ms
 // (1.46), 256^2 x 147 pairs 5.5 ms (6.2).  A whole 512^2 x 100 propagation
