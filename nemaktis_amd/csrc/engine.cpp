@@ -1061,11 +1061,14 @@ Tuning default_tuning(int precision, int Mx, int My, int nprops) {
     // after: 256^2 at 147 pairs 3418 -> 3309, 301 x 203 at 21 pairs 631 -> 554,
     // 400 x 300 at 28 pairs 1639 -> 1503, 128^2 at 14 pairs 161 -> 131, 512^2 at
     // 2 pairs 352 -> 314; a lone pair gains up to 400 points (256^2 109 -> 106)
-    // and loses at 512 (188 -> 191).  Over 120 random meshes and batches the FP32
-    // march is at least 0.993 times as fast as with the shapes before; its error
-    // against FP64, over 91 outputs of 47 jobs that changed shape, 0.98 times
+    // and loses at 512 (188 -> 191).  On x lines above 256 points a few lines do
+    // not pay: a lone pair loses up to 4 % (333 x 51 69.0 -> 71.5), two pairs below
+    // 128 lines 1 to 2 %.  Over 900 meshes and batches the FP32 march is at least
+    // 0.98 times as fast as with the shapes before; its error against FP64, over 91
+    // outputs of 47 jobs that changed shape, is 0.98 times theirs
     const int longest = std::max(Mx, My);
-    const bool lean = precision == 32 && longest <= 512 && (nprops > 2 || longest <= 400);
+    const bool few = Mx > 256 && (nprops <= 2 || (int64_t)My * nprops < 512);
+    const bool lean = precision == 32 && longest <= 512 && !few && (nprops > 2 || longest <= 400);
     const int lcap = precision == 32 && !lean ? 16 : 8;
     if (lean) t.lean = 1;
     auto chunks = [&](int M, int other) {
@@ -1103,8 +1106,10 @@ Tuning default_tuning(int precision, int Mx, int My, int nprops) {
         while (t.y_cols > 1 && (t.y_chunks * t.y_cols > 512 || ylds(t.y_chunks, t.y_cols) > budget)) t.y_cols /= 2;
     // at most 64 blocks leave most CUs idle: half-width strips instead (a lone
     // pair on 256^2 106 -> 100 us a slab, 128^2 74 -> 72; with 76 blocks, 301 x
-    // 203, 112 -> 118)
-    while (precision == 32 && t.y_cols > 4 && (int64_t)((Mx + t.y_cols - 1) / t.y_cols) * nprops <= 64) t.y_cols /= 2;
+    // 203, 112 -> 118), but not of lines under 32 points, whose blocks it brings
+    // down to one wave (222 x 29 55.3 -> 57.3)
+    while (precision == 32 && My >= 32 && t.y_cols > 4 && (int64_t)((Mx + t.y_cols - 1) / t.y_cols) * nprops <= 64)
+        t.y_cols /= 2;
     // slab coefficients on the march stream: as fast or faster than the second
     // stream on every measured batch (up to 12% on small ones, in graph replay)
     t.coef_serial = 1;

@@ -12,6 +12,7 @@ static int last, skip, fail, launches, unfit;
 static size_t live;
 static struct { const void *f; char name[256]; } kernels[4096];
 static int nkernels, seen[4096];
+static unsigned blocks[4096];
 
 /* of the following hipMalloc calls, the first s succeed and the next n fail */
 void stub_fail(int s, int n) { skip = s, fail = n; }
@@ -27,6 +28,7 @@ int stub_seen(int i) {
     seen[i] = 0;
     return v;
 }
+unsigned stub_blocks(int i) { return blocks[i]; } /* of its last launch */
 void **__hipRegisterFatBinary(const void *b) { return (void)b, (void **)kernels; }
 void __hipUnregisterFatBinary(void **b) { (void)b; }
 void __hipRegisterFunction(void **b, const void *f, char *d, const char *name, unsigned n, void *t, void *bl, void *bd,
@@ -65,10 +67,11 @@ int hipFree(void *p) {
     return OK;
 }
 int hipLaunchKernel(const void *f, dim g, dim b, void **args, size_t lds, void *st) {
-    (void)g, (void)b, (void)lds, (void)st;
+    (void)b, (void)lds, (void)st;
     for (int i = 0; i < nkernels; i++)
         if (kernels[i].f == f) {
             seen[i] = 1;
+            blocks[i] = g.x;
             if (strstr(kernels[i].name, "6k_walkI")) { /* WalkMaterial: two orders of the material, the factors */
                 const double **m = args[4];
                 if (!m[0] || !m[1] || !m[2] || m[2][0] != m[2][0]) unfit++;
@@ -77,9 +80,14 @@ int hipLaunchKernel(const void *f, dim g, dim b, void **args, size_t lds, void *
     launches++;
     return OK;
 }
-int __hipPushCallConfiguration(dim g, dim b, size_t lds, void *st) { return (void)g, (void)b, (void)lds, (void)st, OK; }
+static dim grid, block; /* of the launch under way */
+int __hipPushCallConfiguration(dim g, dim b, size_t lds, void *st) {
+    (void)lds, (void)st;
+    grid = g, block = b;
+    return OK;
+}
 int __hipPopCallConfiguration(dim *g, dim *b, size_t *lds, void **st) {
-    g->x = g->y = g->z = b->x = b->y = b->z = 1;
+    *g = grid, *b = block;
     *lds = 0;
     *st = NULL;
     return OK;

@@ -53,6 +53,21 @@ ROUTES = [
     ((3, 65), 1, 1, 64, False),        # an axis that is not periodic
 ]
 
+# mesh, directions, wavelengths: whether FP32 takes the register-lean solvers.  Fuller / lean, us a slab or rates
+LEAN = [
+    ((257, 257), 1, 1, True),          # 109 / 106
+    ((257, 101), 1, 1, True),
+    ((334, 52), 1, 1, False),          # 69.0 / 71.5
+    ((401, 401), 1, 1, False),         # 1 / 0.99
+    ((200, 401), 1, 1, True),          # 1 / 1.07
+    ((512, 512), 1, 1, False),         # 188 / 191
+    ((401, 102), 1, 2, False),         # 1 / 0.99
+    ((401, 161), 1, 2, True),          # 1 / 1.15
+    ((301, 203), 7, 3, True),          # 631 / 554
+    ((513, 513), 7, 1, True),
+    ((514, 514), 7, 1, False),
+]
+
 DRIVER = """
 import ctypes, json, sys
 stub = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
@@ -71,13 +86,14 @@ for (nx, ny), nq, nwl, precision, _ in json.loads(sys.argv[3]):
     with bpm_backend.Context(json.dumps(s), lc, int(np.prod(fields.output_shape(s))), precision=precision,
                              wl_batch=0) as c:
         c.propagate()
-    names = [stub.stub_name(i).decode() for i in range(stub.stub_kernels()) if stub.stub_seen(i)]
+    names = {stub.stub_name(i).decode(): stub.stub_blocks(i) for i in range(stub.stub_kernels()) if stub.stub_seen(i)}
     print("route", json.dumps(names))
 """
 
 
 def launched(so, jobs):
-    """The mangled names of the library's kernels, and of those that each job launches."""
+    """The mangled names of the library's kernels, and of those that each job launches with the blocks of the last
+    launch."""
     r = subprocess.run([sys.executable, "-c", DRIVER, so, ROOT, json.dumps(jobs)], stdout=subprocess.PIPE,
                        stderr=subprocess.STDOUT, text=True, timeout=600)
     assert r.returncode == 0, r.stdout[-3000:]
@@ -103,6 +119,22 @@ def test_routes(stub):
         assert walks != stored, (job, names)
         got.append(job[:4] + (walks,))
     assert got == ROUTES
+
+
+def test_lean_shapes(stub):
+    got = []
+    for job, names in zip(LEAN, launched(stub, [j[:3] + (32, True) for j in LEAN])[1]):
+        lean = {re.search(r"k_ysolveIfLi\d+ELi[01]ELi([01])E", n).group(1) for n in names if "k_ysolve" in n}
+        assert len(lean) == 1
+        got.append(job[:3] + (lean == {"1"},))
+    assert got == LEAN
+
+
+def test_short_lines_keep_whole_strips(stub):
+    """FP32, a lone pair: strips of lines under 32 points are not halved (222 x 29 55.3 us a slab, halved 57.3)."""
+    short, long = ([b for n, b in names.items() if "k_ysolve" in n][0]
+                   for names in launched(stub, [((222, ny), 1, 1, 32, True) for ny in (29, 33)])[1])
+    assert 2 * short <= long + 8
 
 
 def test_the_library_holds_no_walking_kernel_that_nothing_reaches(stub):
